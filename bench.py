@@ -132,9 +132,9 @@ def build_layers(torch, hip, n_layers, dev, hidden=2048, experts=128, ffn=768):
 
 
 PREFILL_TOKENS = 512
-MFMA_BF16_PEAK_TFLOPS = 2500.0  # dense bf16 MFMA; the prefill GEMMs run on it
+MFMA_BF16_PEAK_TFLOPS = 2500.0  # dense bf16 or fp16 MFMA; the prefill GEMMs run on it
 MFMA_F32_PEAK_TFLOPS = 157.3
-SPLIT_PASSES = 3  # activations as three exact bf16 parts: three MFMA passes per product
+SPLIT_PASSES = 2  # activations as two fp16 halves: two MFMA passes per product
 # 512 tokens x 8 routes x (gate + up + down: 3 x 2 x 2048 x 768 flops) + router 512 x 128 x 2 x 2048
 PREFILL_FLOPS = PREFILL_TOKENS * 8 * 9_437_184 + PREFILL_TOKENS * 128 * 2 * 2048
 PREFILL_GEMM_FLOPS = {"gate_up": PREFILL_TOKENS * 8 * 2 * 2 * 2048 * 768,
@@ -212,10 +212,10 @@ def prefill_leg(torch, hip, layers, stream, reps: int, with_cpu: bool):
         "flops_per_batch": PREFILL_FLOPS,
         "tflops": round(whole_tflops, 2),
         "roofline": {"bound": "mfma",
-                     "kernel": "k_expert_gemm<Q4_K, gate/up> (v_mfma_f32_32x32x16_bf16)",
+                     "kernel": "k_expert_gemm<Q4_K, gate/up> (v_mfma_f32_32x32x16_f16)",
                      "achieved": round(gu_tflops, 2), "peak": MFMA_BF16_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(gu_tflops / MFMA_BF16_PEAK_TFLOPS, 4),
-                     # issued = algorithmic x three bf16 planes x tile padding
+                     # issued = algorithmic x two fp16 halves x tile padding
                      "mfma_issued_tflops": round(SPLIT_PASSES * tile_padding * gu_tflops, 2),
                      "tile_padding": round(tile_padding, 3),
                      "frac_of_fp32_mfma_peak": round(gu_tflops / MFMA_F32_PEAK_TFLOPS, 4),

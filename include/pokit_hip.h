@@ -284,9 +284,9 @@ pk_hip_status pk_hip_moe35_decode_async(pk_hip_ctx* ctx, const pk_hip_moe35_laye
  * states; y [tokens][hidden], ids and probs [tokens][top_k] receive each
  * token's moe_result and routes, equal to pk_hip_moe_decode's for that token
  * (ids bit-exact, outputs within FP32 reassociation).  Tokens are grouped per
- * expert; the expert products run on bf16 MFMA with exact products (FP32
- * activations split into three bf16 parts, the quantised weights as exact
- * bf16 integers, scales applied per group in FP32).  1 <= tokens <=
+ * expert; the expert products run on fp16 MFMA (FP32 activations as two fp16
+ * halves under a power-of-two scale per row, the quantised weights as exact
+ * fp16 integers, the remaining scales applied in FP32).  1 <= tokens <=
  * 4096; gate/up and down of any K-quant/Q8_0/Q4_0/Q4_1 type, ffn a multiple of
  * 256.  Host buffers; synchronous.  Non-finite router logits return
  * RUNTIME_ERROR. */

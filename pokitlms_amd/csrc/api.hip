@@ -170,7 +170,7 @@ struct pk_hip_ctx {
     DeviceBuffer<double> row_sum, row_bound;
     DeviceBuffer<float> mvpart;  // the K-sliced batched matvec's slice sums
     // prefill scratch (grown on demand)
-    DeviceBuffer<float> px, py, pprobs, pout, pxsum, pasum;
+    DeviceBuffer<float> px, py, pprobs, pout, pxsum, pasum, pxscale, pascale;
     DeviceBuffer<uint32_t> pids, poffsets, ptiles, pperm;
     DeviceBuffer<uint16_t> pxparts, paparts;
     DeviceBuffer<double> prow_sum, prow_bound;
@@ -641,7 +641,8 @@ void pk_hip_destroy(pk_hip_ctx* c) {
     c->row_sum.release();
     c->row_bound.release();
     c->mvpart.release();
-    for (auto* b : {&c->px, &c->py, &c->pprobs, &c->pout, &c->pxsum, &c->pasum})
+    for (auto* b : {&c->px, &c->py, &c->pprobs, &c->pout, &c->pxsum, &c->pasum, &c->pxscale,
+                    &c->pascale})
         b->release();
     for (auto* b : {&c->pids, &c->poffsets, &c->ptiles, &c->pperm}) b->release();
     c->pxparts.release();
@@ -1101,10 +1102,12 @@ void enqueue_prefill(pk_hip_ctx* c, const pk_hip_moe_layer* L, const MoeShape& m
     c->poffsets.ensure(E + 1);
     c->ptiles.ensure(static_cast<size_t>(max_tiles) + 1);
     c->pperm.ensure(T * K);
-    c->pxparts.ensure(3 * T * m.hidden);
-    c->pxsum.ensure(T * m.hidden / 16);
-    c->paparts.ensure(3 * T * K * m.ffn);
-    c->pasum.ensure(T * K * m.ffn / 16);
+    c->pxparts.ensure(2 * T * m.hidden);
+    c->pxsum.ensure(T * m.hidden / 32);
+    c->pxscale.ensure(T);
+    c->paparts.ensure(2 * T * K * m.ffn);
+    c->pasum.ensure(T * K * m.ffn / 32);
+    c->pascale.ensure(T * K * m.ffn / 32);
     c->pout.ensure(T * K * m.hidden);
     pk::MoePrefillArgs a{};
     pk::MoeDecodeArgs& l = a.layer;
@@ -1149,8 +1152,10 @@ void enqueue_prefill(pk_hip_ctx* c, const pk_hip_moe_layer* L, const MoeShape& m
     a.perm = c->pperm.ptr;
     a.x_parts = c->pxparts.ptr;
     a.x_sums = c->pxsum.ptr;
+    a.x_scale = c->pxscale.ptr;
     a.act_parts = c->paparts.ptr;
     a.act_sums = c->pasum.ptr;
+    a.act_scale = c->pascale.ptr;
     a.out = c->pout.ptr;
     a.status = status_words(c);
     if (c->time_kernels) hold_stream(c, s);

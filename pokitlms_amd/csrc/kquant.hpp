@@ -808,12 +808,6 @@ __device__ __forceinline__ void bf16_bytes(uint32_t w, uint32_t& lo, uint32_t& h
     hi = bf16_pair(ub<2>(w), ub<3>(w));
 }
 
-// bf16 bits of a finite x, rounded to nearest even.
-__device__ __forceinline__ uint32_t bf16_rne_bits(float x) {
-    const uint32_t u = __float_as_uint(x);
-    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-}
-
 // The bytes f0..f3 of w as the bf16 pairs of 128 + f (bits 0x4300 | f: the
 // exponent of 128 leaves f in the low mantissa bits), one v_perm per pair:
 // the weight operand of the MFMA kernels, whose group bias absorbs the

@@ -100,11 +100,12 @@ hipError_t launch_moe_decode(const MoeDecodeArgs& a, hipStream_t stream);
 // Batched prefill: tokens independent single-token MoE blocks, grouped per
 // expert for MFMA GEMMs.  Scratch sizes for `tokens` tokens (T), top_k (K),
 // n_experts (E), pairs P = T*K: row_sum/row_bound T*E, offsets E+1, tiles and
-// n_tiles moe_prefill_max_tiles(T, K, E) + 1, perm P, x_parts 3*T*hidden,
-// x_sums T*hidden/16, act_parts 3*P*ffn, act_sums P*ffn/16,
-// out P*hidden.  Variant 1 (Qwen3.5) adds the shared expert as one more
-// route per token and one more router row and expert group: K = top_k + 1 and
-// E = n_experts + 1 in these sizes.
+// n_tiles moe_prefill_max_tiles(T, K, E) + 1, perm P, x_parts 2*T*hidden,
+// x_sums T*hidden/32, x_scale T, act_parts 2*P*ffn, act_sums and act_scale
+// P*ffn/32, out P*hidden.  Variant 1 (Qwen3.5) adds the shared expert as one
+// more route per token and one more router row and expert group: K = top_k + 1
+// and E = n_experts + 1 in these sizes.
+constexpr uint32_t kGemmTileM = 64;  // assignments per GEMM tile (32 when an expert has no more left)
 constexpr uint32_t kMaxPrefillTokens = 4096;
 struct MoePrefillArgs {
     MoeDecodeArgs layer;     // weights, shapes, top_k, normalize, scale
@@ -119,10 +120,13 @@ struct MoePrefillArgs {
     uint32_t* tiles;         // [max_tiles]
     uint32_t* n_tiles;       // [1]
     uint32_t* perm;          // [P]: grouped row -> token * top_k + route
-    uint16_t* x_parts;       // 3 bf16 planes [tokens][hidden]: x = hi + mid + lo
-    float* x_sums;           // [tokens][hidden / G]: sums over gate/up scale groups
-    uint16_t* act_parts;     // 3 bf16 planes [P][ffn], grouped rows (gate/up epilogue)
-    float* act_sums;         // [P][ffn / G]: sums over down scale groups
+    // the GEMMs' operands (gemm_split.hpp): fp16 halves [row][stage of 32][hi, lo][32]
+    uint16_t* x_parts;       // [tokens]
+    float* x_sums;           // [tokens][hidden / 32]: sums of 32 values
+    float* x_scale;          // [tokens]: the row's power-of-two scale
+    uint16_t* act_parts;     // [P], grouped rows (gate/up epilogue)
+    float* act_sums;         // [P][ffn / 32], where the down format has mins
+    float* act_scale;        // [P][ffn / 32]: each stage's scale
     float* out;              // [P][hidden], slot token * top_k + route
     uint32_t* status;        // as MoeDecodeArgs::status
 };
@@ -135,6 +139,9 @@ bool moe_prefill_supported(uint32_t gate_type, uint32_t up_type, uint32_t down_t
 hipError_t launch_prefill_routing(const MoePrefillArgs& a, hipStream_t stream);
 hipError_t launch_prefill_gate_up(const MoePrefillArgs& a, hipStream_t stream);
 hipError_t launch_prefill_down(const MoePrefillArgs& a, hipStream_t stream);
+// The grouped GEMMs alone (expert_gemm.hip).
+hipError_t launch_expert_gate_up(const MoePrefillArgs& a, hipStream_t stream);
+hipError_t launch_expert_down(const MoePrefillArgs& a, hipStream_t stream);
 
 // Whole-model greedy decode (Qwen3-MoE).  One step = one token through every
 // layer; the step's position and token are read from `state` and `tokens` in

@@ -1,0 +1,83 @@
+"""The prefill's expert GEMMs at the edges of their tiles and number formats.
+
+Expert groups of exactly 1 to 130 rows (tiles hold 64 assignments, or 32 where
+an expert has no more left), every weight format, blocks whose scales are zero
+(Q4_K keeps its accumulator in units of the block's d), and activations over a
+wide range (each row is split into fp16 pairs under its own scale), through
+pk_hip_moe_prefill against the CPU oracle.
+
+Tolerance: both sides sum at most 512 FP32 products twice; a random walk of
+roundings is 512**0.5 * 2**-24 = 1.4e-6 per sum and side, times about four where
+quants and mins are summed apart: 1e-5 normwise.
+"""
+import numpy as np
+import pytest
+
+from pokitlms_amd import synth as S
+from tests.conftest import normwise_rel
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+GROUPS = (1, 31, 32, 33, 63, 64, 65, 130)
+QUANT = (S.Q4_0, S.Q4_1, S.Q8_0, S.Q4_K, S.Q5_K, S.Q6_K)
+HIDDEN, FFN = 512, 256
+
+
+def grouped_layer(gate_type, down_type, seed):
+    """A top-1 layer whose expert e takes the tokens with x[e] large, and its
+    tokens: GROUPS[e] of them, shuffled."""
+    E = len(GROUPS)
+    layer = S.moe_layer(seed=seed, hidden=HIDDEN, experts=E, ffn=FFN, top_k=1,
+                        gate_type=gate_type, up_type=gate_type, down_type=down_type)
+    layer.router = np.zeros((E, HIDDEN), np.float32)
+    layer.router[np.arange(E), np.arange(E)] = 1.0
+    g = S.rng(seed + 1)
+    who = g.permutation(np.repeat(np.arange(E), GROUPS))
+    x = S.normal_f32(g, who.size * HIDDEN).reshape(who.size, HIDDEN)
+    x[np.arange(who.size), who] = 30.0
+    return layer, x, who
+
+
+def check(hip, port, layer, x, who, tokens):
+    h = hip.upload_moe_layer(layer)
+    y, ids, _ = hip.moe_prefill(h, x)
+    h.release()
+    assert np.array_equal(ids[:, 0], who)
+    blk = port.moe(layer)
+    for t in tokens:
+        cy = blk.forward(x[t])[0]
+        assert np.all(np.isfinite(y[t])) and normwise_rel(y[t], cy) <= TOL, (t, who[t])
+
+
+@pytest.mark.parametrize("gtype", QUANT, ids=lambda t: S.TYPE_NAMES[t])
+def test_group_sizes(hip, port, gtype):
+    layer, x, who = grouped_layer(gtype, gtype, 900 + gtype)
+    check(hip, port, layer, x, who, range(0, who.size, 3))
+
+
+@pytest.mark.parametrize("gtype", (S.Q4_K, S.Q5_K), ids=lambda t: S.TYPE_NAMES[t])
+def test_zero_and_spread_block_scales(hip, port, gtype):
+    """d zero in the first, the last, or both blocks of a row, dmin zero or not,
+    and d five decades apart between neighbouring blocks."""
+    layer, x, who = grouped_layer(gtype, gtype, 950 + gtype)
+    for name in ("gate", "up", "down"):
+        w = getattr(layer, name)
+        b = w.reshape(-1, S.BLOCK_BYTES[gtype])
+        n = np.arange(b.shape[0])
+        b[n % 7 == 0, 0:2] = 0
+        b[n % 5 == 1, 0:2] = 0
+        b[n % 11 == 3, 2:4] = 0
+        tiny = np.float16(1e-6).reshape(1).view(np.uint8)
+        b[n % 6 == 2, 0:2] = tiny
+    check(hip, port, layer, x, who, range(0, who.size, 5))
+
+
+def test_activation_range(hip, port):
+    """Rows scaled by 1e-12 to 1e12, and values far below their row's maximum."""
+    layer, x, who = grouped_layer(S.Q4_K, S.Q6_K, 970)
+    x[:, 64:] *= np.float32(2.0) ** -np.arange(0, 28).repeat(16).astype(np.float32)
+    scale = np.float32(10.0) ** (np.arange(who.size) % 13 - 6).astype(np.float32)
+    x *= scale[:, None]
+    layer.router *= np.float32(1e-3)
+    check(hip, port, layer, x, who, range(0, who.size, 2))
