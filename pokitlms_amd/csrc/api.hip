@@ -1140,6 +1140,7 @@ void enqueue_prefill(pk_hip_ctx* c, const pk_hip_moe_layer* L, const MoeShape& m
     }
     a.tokens = tokens;
     a.max_tiles = max_tiles;
+    a.tile_wgs = pk::moe_prefill_tile_wgs(m.hidden, m.ffn);
     a.x = dx;
     a.y = dy;
     a.ids = dids;

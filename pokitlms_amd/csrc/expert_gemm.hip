@@ -13,8 +13,10 @@
 // Q4_K's scales go into the integers instead of one FMA per element and group,
 // and the K order inside a group is the one the masks leave.  Against 32-row
 // tiles of three bf16 parts with 128-biased weights, hidden 2048, ffn 768, 128
-// experts, top-8, Q4_K / Q6_K: 4096 tokens gate/up 918 -> 526 us, down 636 ->
-// 412 us; 512 tokens (skewed load) 193 -> 141 and 141 -> 103 us.  Error against
+// experts, top-8, Q4_K / Q6_K: 4096 tokens gate/up 918 -> 472 us, down 636 ->
+// 403 us; 512 tokens (skewed load) 193 -> 118 and 141 -> 103 us.  (Loads of weights
+// as whole lines through LDS, fragments read half a step ahead with a barrier
+// every second step, and both: the same gate/up time, slower down.)  Error against
 // float64 on the same inputs, before and after: Q4_K/Q6_K 3.8e-6 -> 7.8e-7,
 // Q6_K 9.7e-7 -> 3.6e-7, Q5_K 4.4e-7 -> 4.0e-7, Q8_0 4.4e-7 -> 3.0e-7, Q4_0
 // 4.4e-7 -> 2.9e-7, Q4_1 4.4e-7 -> 4.0e-7.
@@ -373,8 +375,9 @@ __device__ __forceinline__ bool tile_ref(const MoePrefillArgs& a, uint32_t tile,
     r.e = code >> 16;
     const uint32_t lo = __builtin_amdgcn_readfirstlane(a.offsets[r.e]);
     const uint32_t hi = __builtin_amdgcn_readfirstlane(a.offsets[r.e + 1]);
-    r.base = lo + (code & 0xffffu) * kGemmTileM;
-    r.rows = hi - r.base < kGemmTileM ? hi - r.base : kGemmTileM;
+    r.base = lo + (code & 0x7fffu) * 32u;
+    const uint32_t most = code & kTileBig ? kGemmTileM : 32u;
+    r.rows = hi - r.base < most ? hi - r.base : most;
     return true;
 }
 
@@ -399,15 +402,17 @@ struct GemmShared {
     float scale[kGemmTileM];
 };
 
-// Maximum of |v| over each 32-lane half, in all its lanes.
+// Maximum of |v| over each 32-lane half, in all its lanes (as unsigned bits, whose
+// zero identity lets each DPP step fold into the maximum; NaN sorts last and
+// gives the scale of an infinity).
 __device__ __forceinline__ float half_wave_max(float v) {
-    v = fmaxf(v, dpp<0xb1>(v));
-    v = fmaxf(v, dpp<0x4e>(v));
-    v = fmaxf(v, dpp<0x141>(v));
-    v = fmaxf(v, dpp<0x140>(v));
-    const uint32_t u = __float_as_uint(v);
+    uint32_t u = __float_as_uint(v) & 0x7fffffffu;
+    u = max(u, dpp_u0max<0xb1>(u));
+    u = max(u, dpp_u0max<0x4e>(u));
+    u = max(u, dpp_u0max<0x141>(u));
+    u = max(u, dpp_u0max<0x140>(u));
     const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    return fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
+    return __uint_as_float(max(s[0], s[1]));
 }
 
 // MT x 32 assignments of a tile, from its row row0.  DUAL: gate and up rows n0 .. n0 + 127 over x,
@@ -462,8 +467,12 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         csrc[i] = DUAL ? nullptr : a.act_scale + static_cast<uint64_t>(sh.arow[row0 + row]) * nst;
         cinv[i] = DUAL ? 0.0f : 1.0f / sh.scale[row0 + row];
     }
-    u32x4_t av[2][MT];
-    float ac[2][MT];
+    // register sets of stages in flight: with one row block there is room for eight,
+    // which small batches need, where little else hides the loads' latency (77
+    // tokens, 64 experts: gate/up 45 -> 42 us; 512 tokens 119 -> 117)
+    constexpr uint32_t NS = MT == 1 ? 8u : 2u;
+    u32x4_t av[NS][MT];
+    float ac[NS][MT];
     const uint32_t last = nst - 1u;
     auto load_act = [&](uint32_t set, uint32_t s) {  // past the end: the last stage again
         const uint32_t st = s < last ? s : last;
@@ -521,10 +530,11 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
 
     load_act(0u, 0u);
     load_sums(0u);
-    load_act(1u, 1u);
+#pragma unroll
+    for (uint32_t i = 1; i < NS; ++i) load_act(i, i);
     store_act(0u, 0u);
     store_sums(0u);
-    load_act(0u, 2u);
+    load_act(0u, NS);
     __syncthreads();
 
     f32x16 acc[MT][2], part[MT][2];  // part: Q5_K, the superblock's sums
@@ -632,8 +642,8 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
             }
 #pragma unroll
             for (uint32_t i = 0; i < 2; ++i) wreload<T>(ws[i], blk, sb, bn, j, kq, raw[i]);
-            store_act(buf ^ 1u, buf ^ 1u);
-            load_act(buf ^ 1u, s + 3u);
+            store_act((j + 1u) % NS, buf ^ 1u);
+            load_act((j + 1u) % NS, s + 1u + NS);
             if (j == 4u) store_sums(sbuf ^ 1u);
             __syncthreads();
         }
@@ -642,34 +652,42 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     // results: the accumulators' units are d 2^24 s (kSuper) or s (the row's scale)
     const float u0 = W::kUnits ? dcur[0] * 0x1p24f : 1.0f, u1 = W::kUnits ? dcur[1] * 0x1p24f : 1.0f;
     if constexpr (DUAL) {
-        // SwiGLU g / (1 + expf(-g)) * u (src/qwen3_moe_runner.cpp:682-684); variant 1:
-        // silu(g) * u (src/qwen35_runner.cpp:111-123), and the values split as the
-        // down GEMM's operands: the wave's 32 columns of a row are one chunk.
+        // SwiGLU g / (1 + exp(-g)) * u (src/qwen3_moe_runner.cpp:682-684, and variant 1's
+        // silu(g) * u, src/qwen35_runner.cpp:111-123) with the hardware exp2 and
+        // reciprocal, as the decode path; the values split as the down GEMM's
+        // operands: the wave's 32 columns of a row are one chunk.  (With the libm
+        // expf, IEEE division and 64-bit addresses this part took nearly half of
+        // the kernel's vector instructions: 526 -> 494 us at 4096 tokens.)
         const uint32_t col = n0 + wave * 32u + ln, chunk = col / 32u, nch = ndim / 32u;
         const uint32_t at = (ln & 24u) | kPairOrder(ln & 7u);
         const bool dmins = L.down_type == T_Q4_K || L.down_type == T_Q5_K || L.down_type == T_Q4_1;
+        // this lane's place in row 0 of the tile's rows; rows are nch stages apart
+        const uint64_t rc0 = static_cast<uint64_t>(tr.base) * nch + chunk;
+        uint16_t* pd = a.act_parts + rc0 * 64u + at;
+        float* cd = a.act_scale + rc0;
+        float* sd = a.act_sums + rc0;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
 #pragma unroll
             for (uint32_t r = 0; r < 16; ++r) {
                 const uint32_t row = row0 + 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
                 const float s = sh.scale[row];
-                const float g = acc[m][0][r] * u0 * s, u = acc[m][1][r] * u1 * s;
-                const float v = L.variant ? silu(g) * u : (g / (1.0f + expf(-g))) * u;
+                const float g = acc[m][0][r] * (u0 * s), u = acc[m][1][r] * (u1 * s);
+                const float v = (g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))) * u;
                 float cs, cinv2;
-                split_scale(half_wave_max(fabsf(v)), cs, cinv2);
+                split_scale(half_wave_max(v), cs, cinv2);
                 const float w = v * cinv2;
                 const _Float16 h = static_cast<_Float16>(w);
                 const _Float16 l = static_cast<_Float16>(w - static_cast<float>(h));
-                double gs = 0.0;
-                if (dmins) gs = group_sum<32>(static_cast<double>(v));  // uniform
+                float gs = 0.0f;
+                if (dmins) gs = static_cast<float>(group_sum<32>(static_cast<double>(v)));  // uniform
                 if (row < tr.rows) {
-                    const uint64_t rc = static_cast<uint64_t>(tr.base + row) * nch + chunk;
-                    a.act_parts[rc * 64u + at] = __builtin_bit_cast(uint16_t, h);
-                    a.act_parts[rc * 64u + 32u + at] = __builtin_bit_cast(uint16_t, l);
+                    const uint32_t off = row * nch;
+                    pd[off * 64u] = __builtin_bit_cast(uint16_t, h);
+                    pd[off * 64u + 32u] = __builtin_bit_cast(uint16_t, l);
                     if (ln == 31u) {
-                        a.act_scale[rc] = cs;
-                        if (dmins) a.act_sums[rc] = static_cast<float>(gs);
+                        cd[off] = cs;
+                        if (dmins) sd[off] = gs;
                     }
                 }
             }
@@ -755,6 +773,10 @@ hipError_t expert_gemm(uint32_t type, const MoePrefillArgs& a, hipStream_t s) {
 }
 
 }  // namespace
+
+uint32_t moe_prefill_tile_wgs(uint32_t hidden, uint32_t ffn) {
+    return ffn / kRowsN > hidden / (2u * kRowsN) ? ffn / kRowsN : hidden / (2u * kRowsN);
+}
 
 hipError_t launch_expert_gate_up(const MoePrefillArgs& a, hipStream_t s) {
     return expert_gemm<true>(a.layer.gate_type, a, s);

@@ -105,11 +105,15 @@ hipError_t launch_moe_decode(const MoeDecodeArgs& a, hipStream_t stream);
 // P*ffn/32, out P*hidden.  Variant 1 (Qwen3.5) adds the shared expert as one
 // more route per token and one more router row and expert group: K = top_k + 1
 // and E = n_experts + 1 in these sizes.
-constexpr uint32_t kGemmTileM = 64;  // assignments per GEMM tile (32 when an expert has no more left)
+constexpr uint32_t kGemmTileM = 64;   // assignments per GEMM tile (32 when an expert has no more left)
+constexpr uint32_t kGemmSlots = 512;  // GEMM workgroups the chip holds at once: two per CU
+// A tile: expert << 16 | kTileBig (64 rows, else 32) | first row / 32 in the expert's group.
+constexpr uint32_t kTileBig = 1u << 15;
 constexpr uint32_t kMaxPrefillTokens = 4096;
 struct MoePrefillArgs {
     MoeDecodeArgs layer;     // weights, shapes, top_k, normalize, scale
     uint32_t tokens, max_tiles;
+    uint32_t tile_wgs;       // GEMM workgroups per tile, the larger of gate/up's and down's
     const float* x;          // [tokens][hidden]
     float* y;                // [tokens][hidden]
     uint32_t* ids;           // [tokens][top_k]
@@ -130,6 +134,7 @@ struct MoePrefillArgs {
     float* out;              // [P][hidden], slot token * top_k + route
     uint32_t* status;        // as MoeDecodeArgs::status
 };
+uint32_t moe_prefill_tile_wgs(uint32_t hidden, uint32_t ffn);
 uint32_t moe_prefill_max_tiles(uint32_t tokens, uint32_t top_k, uint32_t n_experts);
 bool moe_prefill_supported(uint32_t gate_type, uint32_t up_type, uint32_t down_type,
                            uint32_t hidden, uint32_t ffn, uint32_t n_experts, uint32_t top_k,

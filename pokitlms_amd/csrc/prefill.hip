@@ -202,6 +202,20 @@ __device__ __forceinline__ void split_row(const float* __restrict__ x, uint32_t 
 
 constexpr uint32_t kGroupThreads = 1024;
 
+// Tiles of an expert with c rows: 64-row ones (the last may hold 33 to 64), and one
+// of at most 32 rows for what is left; or, when that makes no more workgroups
+// than the chip holds at once (kGemmSlots), 32-row tiles only, since the longest
+// workgroup then sets the time (77 tokens, 64 experts and a shared one: gate/up
+// 42 -> 33 us).  The list holds every 64-row tile first, so the GEMMs' longest
+// workgroups start first and short ones fill the tail (512 tokens, skewed load:
+// gate/up 128 -> 119 us).
+__device__ __forceinline__ uint32_t big_tiles(uint32_t c, bool split) {
+    return split ? 0u : c / 64u + (c % 64u > 32u ? 1u : 0u);
+}
+__device__ __forceinline__ uint32_t small_tiles(uint32_t c, bool split) {
+    return split ? (c + 31u) / 32u : (c % 64u > 0u && c % 64u <= 32u) ? 1u : 0u;
+}
+
 // Workgroup 0 groups; the others split x into the gate/up GEMM's operands, a
 // row per wave, while it does, since the grouping alone would leave the rest of
 // the chip idle.
@@ -215,7 +229,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_group(MoePrefillArgs a) {
         return;
     }
     constexpr uint32_t NE = kMaxExperts + 1;  // + the shared expert (variant 1)
-    __shared__ uint32_t cnt[NE], off[NE + 1], tb[NE + 1], fill[NE];
+    __shared__ uint32_t cnt[NE], off[NE + 1], tb[NE], ts[NE], fill[NE], split32;
     const uint32_t E = a.layer.n_experts, K = a.layer.top_k, V = a.layer.variant, tid = threadIdx.x;
     const uint32_t EE = E + V, KR = K + V, n = a.tokens * K;
     if (tid < EE) {
@@ -234,39 +248,52 @@ __global__ __launch_bounds__(kGroupThreads) void k_group(MoePrefillArgs a) {
     __syncthreads();
     if (tid < 64) {  // exclusive prefix of rows and tiles: PER experts a lane, one wave scan
         constexpr uint32_t PER = (NE + 63u) / 64u;
-        uint32_t c[PER], tl[PER];
-        double lc = 0.0, lt = 0.0;  // integer sums, exact in FP64
+        uint32_t c[PER];
+        double l32 = 0.0;  // integer sums, exact in FP64
 #pragma unroll
         for (uint32_t k = 0; k < PER; ++k) {
             const uint32_t e = tid * PER + k;
             c[k] = e < EE ? cnt[e] : 0u;
-            tl[k] = (c[k] + kGemmTileM - 1u) / kGemmTileM;
-            lc += static_cast<double>(c[k]);
-            lt += static_cast<double>(tl[k]);
+            l32 += static_cast<double>(small_tiles(c[k], true));
         }
-        const double ic = wave_inclusive_scan(lc), it = wave_inclusive_scan(lt);
+        const uint32_t t32 = static_cast<uint32_t>(lane63(wave_inclusive_scan(l32)));
+        const bool split = t32 * a.tile_wgs <= kGemmSlots;  // uniform
+        double lc = 0.0, lt = 0.0, ls = 0.0;
+#pragma unroll
+        for (uint32_t k = 0; k < PER; ++k) {
+            lc += static_cast<double>(c[k]);
+            lt += static_cast<double>(big_tiles(c[k], split));
+            ls += static_cast<double>(small_tiles(c[k], split));
+        }
+        const double ic = wave_inclusive_scan(lc), it = wave_inclusive_scan(lt), is = wave_inclusive_scan(ls);
         uint32_t o = static_cast<uint32_t>(ic - lc), b = static_cast<uint32_t>(it - lt);
+        uint32_t sm = static_cast<uint32_t>(lane63(it)) + static_cast<uint32_t>(is - ls);
 #pragma unroll
         for (uint32_t k = 0; k < PER; ++k) {
             const uint32_t e = tid * PER + k;
             if (e < EE) {
                 off[e] = o;
                 tb[e] = b;
+                ts[e] = sm;
             }
             o += c[k];
-            b += tl[k];
+            b += big_tiles(c[k], split);
+            sm += small_tiles(c[k], split);
         }
         if (tid == 63u) {
             off[EE] = static_cast<uint32_t>(ic);
-            tb[EE] = static_cast<uint32_t>(it);
-            a.n_tiles[0] = static_cast<uint32_t>(it);
+            a.n_tiles[0] = static_cast<uint32_t>(it) + static_cast<uint32_t>(is);
+            split32 = split ? 1u : 0u;
         }
     }
     __syncthreads();
     if (tid <= EE) a.offsets[tid] = off[tid];
-    if (tid < EE)
-        for (uint32_t j = 0; j < (cnt[tid] + kGemmTileM - 1u) / kGemmTileM; ++j)
-            a.tiles[tb[tid] + j] = (tid << 16) | j;
+    if (tid < EE) {
+        const bool split = split32 != 0u;
+        const uint32_t nb = big_tiles(cnt[tid], split), ns = small_tiles(cnt[tid], split);
+        for (uint32_t j = 0; j < nb; ++j) a.tiles[tb[tid] + j] = (tid << 16) | kTileBig | (2u * j);
+        for (uint32_t j = 0; j < ns; ++j) a.tiles[ts[tid] + j] = (tid << 16) | (2u * nb + j);
+    }
     // grouped rows hold slots token * (top_k + variant) + route (the shared
     // expert is route top_k); the order inside a group is free: every row's
     // result is independent
@@ -336,7 +363,10 @@ uint32_t ceil_div_u(uint32_t a, uint32_t b) { return (a + b - 1u) / b; }
 
 uint32_t moe_prefill_max_tiles(uint32_t tokens, uint32_t top_k, uint32_t n_experts) {
     const uint32_t pairs = tokens * top_k;
-    return pairs / kGemmTileM + (n_experts < pairs ? n_experts : pairs);
+    // 64-row tiles, one partly filled per expert, or fewer 32-row tiles than kGemmSlots
+    const uint32_t touched = n_experts < pairs ? n_experts : pairs;
+    const uint32_t t64 = pairs / kGemmTileM + touched, t32 = pairs / 32u + touched;
+    return t64 > kGemmSlots ? t64 : t32 < kGemmSlots ? t32 : kGemmSlots;
 }
 
 bool moe_prefill_supported(uint32_t gate_type, uint32_t up_type, uint32_t down_type,

@@ -1,13 +1,14 @@
 """The prefill's expert GEMMs at the edges of their tiles and number formats.
 
 Expert groups of exactly 1 to 130 rows (tiles hold 64 assignments, or 32 where
-an expert has no more left), every weight format, blocks whose scales are zero
+an expert has no more left; only 32 while that makes few workgroups, so once
+with eight experts and once with sixty-four), every weight format, blocks whose scales are zero
 (Q4_K keeps its accumulator in units of the block's d), and activations over a
 wide range (each row is split into fp16 pairs under its own scale), through
 pk_hip_moe_prefill against the CPU oracle.
 
-Tolerance: both sides sum at most 512 FP32 products twice; a random walk of
-roundings is 512**0.5 * 2**-24 = 1.4e-6 per sum and side, times about four where
+Tolerance: both sides sum at most 1024 FP32 products twice; a random walk of
+roundings is 1024**0.5 * 2**-24 = 1.9e-6 per sum and side, times about four where
 quants and mins are summed apart: 1e-5 normwise.
 """
 import numpy as np
@@ -21,20 +22,20 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-5
 GROUPS = (1, 31, 32, 33, 63, 64, 65, 130)
 QUANT = (S.Q4_0, S.Q4_1, S.Q8_0, S.Q4_K, S.Q5_K, S.Q6_K)
-HIDDEN, FFN = 512, 256
 
 
-def grouped_layer(gate_type, down_type, seed):
+def grouped_layer(gate_type, down_type, seed, repeat=1, hidden=512, ffn=256):
     """A top-1 layer whose expert e takes the tokens with x[e] large, and its
-    tokens: GROUPS[e] of them, shuffled."""
-    E = len(GROUPS)
-    layer = S.moe_layer(seed=seed, hidden=HIDDEN, experts=E, ffn=FFN, top_k=1,
+    tokens: GROUPS[e % 8] of them, shuffled."""
+    groups = GROUPS * repeat
+    E = len(groups)
+    layer = S.moe_layer(seed=seed, hidden=hidden, experts=E, ffn=ffn, top_k=1,
                         gate_type=gate_type, up_type=gate_type, down_type=down_type)
-    layer.router = np.zeros((E, HIDDEN), np.float32)
+    layer.router = np.zeros((E, hidden), np.float32)
     layer.router[np.arange(E), np.arange(E)] = 1.0
     g = S.rng(seed + 1)
-    who = g.permutation(np.repeat(np.arange(E), GROUPS))
-    x = S.normal_f32(g, who.size * HIDDEN).reshape(who.size, HIDDEN)
+    who = g.permutation(np.repeat(np.arange(E), groups))
+    x = S.normal_f32(g, who.size * hidden).reshape(who.size, hidden)
     x[np.arange(who.size), who] = 30.0
     return layer, x, who
 
@@ -56,11 +57,19 @@ def test_group_sizes(hip, port, gtype):
     check(hip, port, layer, x, who, range(0, who.size, 3))
 
 
+@pytest.mark.parametrize("gtype", QUANT, ids=lambda t: S.TYPE_NAMES[t])
+def test_group_sizes_many_experts(hip, port, gtype):
+    """136 tiles of 32 rows times four workgroups each are more than 512, so tiles
+    hold 64 rows."""
+    layer, x, who = grouped_layer(gtype, gtype, 910 + gtype, repeat=8, hidden=1024, ffn=512)
+    check(hip, port, layer, x, who, range(0, who.size, 23))
+
+
 @pytest.mark.parametrize("gtype", (S.Q4_K, S.Q5_K), ids=lambda t: S.TYPE_NAMES[t])
 def test_zero_and_spread_block_scales(hip, port, gtype):
     """d zero in the first, the last, or both blocks of a row, dmin zero or not,
     and d five decades apart between neighbouring blocks."""
-    layer, x, who = grouped_layer(gtype, gtype, 950 + gtype)
+    layer, x, who = grouped_layer(gtype, gtype, 950 + gtype, repeat=8, hidden=1024, ffn=512)
     for name in ("gate", "up", "down"):
         w = getattr(layer, name)
         b = w.reshape(-1, S.BLOCK_BYTES[gtype])
@@ -70,7 +79,7 @@ def test_zero_and_spread_block_scales(hip, port, gtype):
         b[n % 11 == 3, 2:4] = 0
         tiny = np.float16(1e-6).reshape(1).view(np.uint8)
         b[n % 6 == 2, 0:2] = tiny
-    check(hip, port, layer, x, who, range(0, who.size, 5))
+    check(hip, port, layer, x, who, range(0, who.size, 29))
 
 
 def test_activation_range(hip, port):
