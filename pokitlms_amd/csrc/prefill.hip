@@ -5,9 +5,8 @@
 // token's routes and output are those of a single-token pass.  Here the
 // whole batch goes through six launches:
 //
-//  1. k_router_batch: the logit value S and rounding bound B of every
-//     (token, expert) pair (the decode router's arithmetic, one expert row
-//     per wave held in registers across a tile of tokens).
+//  1. k_router_batch: the logit value S (the decode router's) and a rounding
+//     bound B of every (token, expert) pair.
 //  2. k_route_batch: one workgroup per token ranks the experts exactly as the
 //     decode path does (certified wave ranking, exact serial fallback) and
 //     writes ids and route weights.
@@ -35,58 +34,173 @@
 namespace pk {
 namespace {
 
-constexpr uint32_t kRouterTokens = 8;  // tokens per batched-router workgroup
-
 // ---------------------------------------------------------------------------
-// 1. Batched router.
+// 1. Batched router: per (token, expert) the value S of the decode router (the
+// FP64 sum of the CPU's rounded FP32 products) and a bound B on the CPU's serial
+// FP32 sum.
+//
+// A workgroup takes 16 tokens x 32 rows; its eight waves split K, and each lane of
+// a wave sums 2 tokens x 4 rows over the wave's range, so a
+// product costs its multiplication, the conversion and one FP64 add, and no
+// scan across lanes is left (one row per wave with a scan and two FP64 adds per
+// product: 275 us for 4096 tokens x 128 rows of 2048, 42 us for 512; so: 116
+// and 21 us, bound by those three instructions; the ranking's second look at what
+// the coarser bound leaves open adds 6 us).  The waves' operands pass
+// through LDS parts of their own; the only barrier is before the waves' sums meet.
+//
+// The bound.  With T_i the exact prefix sums of the products p_i, the serial sum
+// is within u (1 + 2^-10) sum_i |T_i| of S.  In a run of 16 products from prefix O
+// to prefix O', |T_i| <= |O| + the |p| before i in the first half and |O'| + the
+// |p| after i in the second, so the run's sum is at most 8 |O| + 8 |O'| + sum_j
+// o_j |p_j| with o = 8 .. 1, 0 .. 7; and by Cauchy-Schwarz over the whole row
+// sum_j o_j |p_j| <= |o w| |x|, two norms.  A wave's range starts at an offset that
+// the earlier waves' sums give: |O| <= |offset| + |its own prefix|.  On
+// router-like rows of 2048 this is 1.4 times the decode router's bound.
 
-// Expert rows per wave: C = hidden / 256, so 4 * C router values per lane
-// and row stay in registers.
-template <int C>
-constexpr uint32_t router_rows_per_wave() { return C <= 8 ? 4u : C <= 16 ? 2u : 1u; }
+constexpr uint32_t kRtWaves = 8;                        // waves per workgroup, each a range of K
+constexpr uint32_t kRtK = 32, kRtRow = kRtK + 4;        // K per stage; floats per staged row
+struct RouterSums {
+    double l, q;  // a wave's sum, and the sum of its |prefixes| at every 16th product
+};
 
-// Per (token, expert) the S and B of router_wave_sum_bound, from the same
-// lane sums (so the decode path's bits).  Each wave holds R expert rows in
-// registers and walks kRouterTokens tokens, reading each token's x once for
-// its R rows (the next token's x while the current one is summed); the four
-// waves of a workgroup take 4 R rows and the same tokens.  No barrier: the
-// waves never wait for one another.
-template <int C>
-__global__ __launch_bounds__(256) void k_router_batch(MoePrefillArgs a) {
-    constexpr uint32_t R = router_rows_per_wave<C>();
+// Lane (i, j) of a wave takes tokens TT i .. and rows TE j ..: 8 TT tokens x 8 TE
+// rows per workgroup.  2 x 4 where that makes two workgroups per CU, else 1 x 2
+// (a wave's chain is a quarter as long: 512 tokens 33 -> 21 us, 77 tokens x 64
+// rows of 1024 17 -> 6 us).
+template <uint32_t TT, uint32_t TE>
+__global__ __launch_bounds__(64 * kRtWaves, 4) void k_router_batch(MoePrefillArgs a) {
+    constexpr uint32_t T = 8u * TT, R = 8u * TE, NL = TT + TE;
+    __shared__ __attribute__((aligned(16))) union {
+        float stage[kRtWaves][(T + R) * kRtRow];
+        RouterSums part[kRtWaves][T * R];
+    } sh;
+    __shared__ float nx[kRtWaves][T], nw[kRtWaves][R];  // squared norms of each wave's range
     const uint32_t E = a.layer.n_experts, ER = E + a.layer.variant, H = a.layer.hidden;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    // rows: the n_experts router rows, then (variant 1) the shared expert's gate
-    const uint32_t e0 = (blockIdx.x * 4u + wave) * R;
-    const uint32_t t0 = blockIdx.y * kRouterTokens;
-    const uint32_t t1 = t0 + kRouterTokens < a.tokens ? t0 + kRouterTokens : a.tokens;
-    rf32x4 w[R][C], xc[C];
+    const uint32_t e0 = blockIdx.x * R, t0 = blockIdx.y * T;
+    const uint32_t range = H / kRtWaves;  // a multiple of kRtK
+    // staging: piece lane % 8 (4 floats) of rows lane / 8 + 8 i; rows past the end
+    // repeat the last and write nothing
+    const uint32_t pr = lane / 8u, pc = 4u * (lane % 8u);
+    const float* src[NL];
 #pragma unroll
-    for (uint32_t r = 0; r < R; ++r) {
-        const uint32_t ee = e0 + r < ER ? e0 + r : ER - 1u;  // rows past the end repeat the last, write nothing
-        const float* row = ee < E ? a.layer.router + static_cast<uint64_t>(ee) * H : a.layer.shared_router;
-        router_lane_load<C>(row, lane, w[r]);
+    for (uint32_t i = 0; i < NL; ++i) {
+        if (i < TT) {
+            const uint32_t t = t0 + pr + 8u * i < a.tokens ? t0 + pr + 8u * i : a.tokens - 1u;
+            src[i] = a.x + static_cast<uint64_t>(t) * H;
+        } else {
+            const uint32_t e = e0 + pr + 8u * (i - TT) < ER ? e0 + pr + 8u * (i - TT) : ER - 1u;
+            src[i] = e < E ? a.layer.router + static_cast<uint64_t>(e) * H : a.layer.shared_router;
+        }
+        src[i] += wave * range + pc;
     }
-    router_lane_load<C>(a.x + static_cast<uint64_t>(t0) * H, lane, xc);
-    for (uint32_t t = t0; t < t1; ++t) {
-        // the next token's x (the last token reloads its own: unconditional)
-        const uint32_t tn = t + 1u < t1 ? t + 1u : t;
-        rf32x4 xn[C];
-        router_lane_load<C>(a.x + static_cast<uint64_t>(tn) * H, lane, xn);
-        __builtin_amdgcn_sched_barrier(0);  // the loads out before the sums wait
+    // o_j of this lane's four positions in a run of 16, plus 1 (and a little) for the
+    // rounding of the products themselves
+    float om[4];
 #pragma unroll
-        for (uint32_t r = 0; r < R; ++r) {
-            RouterLane<C> rl;
-            double total, bound;
-            router_lane_sums<C>(w[r], xc, rl);
-            router_wave_sum_bound<C>(rl, total, bound);
-            if (lane == 0 && e0 + r < ER) {
-                a.row_sum[static_cast<uint64_t>(t) * ER + e0 + r] = total;
-                a.row_bound[static_cast<uint64_t>(t) * ER + e0 + r] = bound;
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t j = pc % 16u + i;
+        om[i] = (j < 8u ? 8.0f - static_cast<float>(j) : static_cast<float>(j) - 8.0f) + 1.001f;
+    }
+    // stages of loads in flight: two, or one where registers would limit the waves
+    constexpr uint32_t NS = TT == 1u ? 2u : 1u;
+    rf32x4 v[NS][NL];
+    auto load = [&](uint32_t set, uint32_t k) {
+        const uint32_t kk = k < range ? k : range - kRtK;  // past the range: its last stage again
+#pragma unroll
+        for (uint32_t i = 0; i < NL; ++i) v[set][i] = *reinterpret_cast<const rf32x4*>(src[i] + kk);
+    };
+    float* st = sh.stage[wave];
+    float sq[NL];
+#pragma unroll
+    for (uint32_t i = 0; i < NL; ++i) sq[i] = 0.0f;
+    const uint32_t ti = TT * (lane / 8u), ej = TE * (lane % 8u);  // this lane's tokens and rows
+    const float* xr = st + ti * kRtRow;
+    const float* wr = st + (T + ej) * kRtRow;
+    double l[TT][TE], q[TT][TE];
+#pragma unroll
+    for (uint32_t t = 0; t < TT; ++t)
+#pragma unroll
+        for (uint32_t e = 0; e < TE; ++e) l[t][e] = q[t][e] = 0.0;
+#pragma unroll
+    for (uint32_t i = 0; i < NS; ++i) load(i, i * kRtK);
+    auto stage = [&](uint32_t set, uint32_t k) {
+#pragma unroll
+        for (uint32_t i = 0; i < NL; ++i) {
+            *reinterpret_cast<rf32x4*>(st + (pr + 8u * i) * kRtRow + pc) = v[set][i];
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) {
+                const float f = i < TT ? v[set][i][c] : v[set][i][c] * om[c];
+                sq[i] = __builtin_fmaf(f, f, sq[i]);
             }
         }
+        load(set, k + NS * kRtK);
 #pragma unroll
-        for (int j = 0; j < C; ++j) xc[j] = xn[j];
+        for (uint32_t c = 0; c < kRtK / 4u; ++c) {
+            rf32x4 x[TT], w[TE];
+#pragma unroll
+            for (uint32_t t = 0; t < TT; ++t) x[t] = *reinterpret_cast<const rf32x4*>(xr + t * kRtRow + 4u * c);
+#pragma unroll
+            for (uint32_t e = 0; e < TE; ++e) w[e] = *reinterpret_cast<const rf32x4*>(wr + e * kRtRow + 4u * c);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i)
+#pragma unroll
+                for (uint32_t t = 0; t < TT; ++t)
+#pragma unroll
+                    for (uint32_t e = 0; e < TE; ++e)
+                        l[t][e] += static_cast<double>(__fmul_rn(w[e][i], x[t][i]));
+            if (c % 4u == 3u) {
+#pragma unroll
+                for (uint32_t t = 0; t < TT; ++t)
+#pragma unroll
+                    for (uint32_t e = 0; e < TE; ++e) q[t][e] += fabs(l[t][e]);
+            }
+        }
+    };
+    uint32_t k = 0;
+    for (; k + NS * kRtK <= range; k += NS * kRtK)
+#pragma unroll
+        for (uint32_t i = 0; i < NS; ++i) stage(i, k + i * kRtK);
+    if (k < range) stage(0u, k);
+#pragma unroll
+    for (uint32_t i = 0; i < NL; ++i) {
+        const float n = group_sum<8>(sq[i]);
+        if (lane % 8u == 0u) (i < TT ? nx[wave][pr + 8u * i] : nw[wave][pr + 8u * (i - TT)]) = n;
+    }
+    __syncthreads();  // every wave is past its staged operands
+#pragma unroll
+    for (uint32_t t = 0; t < TT; ++t)
+#pragma unroll
+        for (uint32_t e = 0; e < TE; ++e) {
+            RouterSums& p = sh.part[wave][(ti + t) * R + ej + e];
+            p.l = l[t][e];
+            p.q = q[t][e];
+        }
+    __syncthreads();
+    static_assert(T * R <= 64u * kRtWaves, "at most one (token, row) per thread");
+    if (threadIdx.x >= T * R) return;
+    const uint32_t t = threadIdx.x / R, e = threadIdx.x % R;
+    double S = 0.0, Q = 0.0;
+    float xx = 0.0f, ww = 0.0f;
+    const double run = static_cast<double>(range);
+#pragma unroll
+    for (uint32_t w = 0; w < kRtWaves; ++w) {
+        const RouterSums p = sh.part[w][threadIdx.x];
+        // 16 |L| per inner run end, 8 at the range's end, and its offset at both ends of each run
+        Q += 16.0 * p.q - 8.0 * fabs(p.l) + run * fabs(S);
+        S += p.l;
+        xx += nx[w][t];
+        ww += nw[w][e];
+    }
+    // the squares were rounded and summed in FP32 (2^-10 covers it) and may have
+    // underflowed (2^-100 each); router_bound covers the rest, 2^-126 the products
+    // below FP32's range
+    const double slack = 8192.0 * 0x1p-100;
+    const double P = (1.0 + 0x1p-10) * sqrt((static_cast<double>(xx) + slack) * (static_cast<double>(ww) + slack));
+    if (t0 + t < a.tokens && e0 + e < ER) {
+        const uint64_t at = static_cast<uint64_t>(t0 + t) * ER + e0 + e;
+        a.row_sum[at] = S;
+        a.row_bound[at] = router_bound(Q + P) + 0x1p-126;
     }
 }
 
@@ -98,8 +212,8 @@ __global__ __launch_bounds__(256) void k_route_batch(MoePrefillArgs A) {
     extern __shared__ __attribute__((aligned(16))) float xs[];  // [hidden]
     __shared__ FallbackShared<256> fb;
     __shared__ uint32_t s_sel[kMaxTopK];
-    __shared__ uint32_t s_state;
-    __shared__ double s_lo;
+    __shared__ uint32_t s_state, s_ncand, s_cand[kMaxExperts];
+    __shared__ double s_lo, s_S[kMaxExperts], s_B[kMaxExperts];
     const uint32_t t = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t E = A.layer.n_experts, K = A.layer.top_k;
     MoeDecodeArgs a = A.layer;  // this token's view
@@ -115,24 +229,66 @@ __global__ __launch_bounds__(256) void k_route_batch(MoePrefillArgs A) {
     if (wave == 0) rd = load_route_data<NS>(a);
     store_x_regs(xs, xr, a.hidden);
     WaveRoutes<NS> w;
-    if (wave == 0) {
+    auto rank = [&] {  // wave 0
         w = wave_route<NS>(a, rd);
         if (lane == 0) {
 #pragma unroll
             for (uint32_t r = 0; r < kMaxTopK; ++r) s_sel[r] = w.sel[r];
             s_state = !w.finite ? 2u : w.certified ? 0u : 1u;
             s_lo = w.lo_min_sel;
+            s_ncand = 0u;
         }
-    }
+    };
+    if (wave == 0) rank();
     __syncthreads();
-    const uint32_t state = s_state;  // uniform
+    uint32_t state = s_state;  // uniform
+    if (state == 1u) {
+        // The batched router's bound does not certify the ranking: form the decode
+        // router's sum and bound of every expert whose interval reaches the selected
+        // ones, and rank again.  An expert below them by the coarser bound is below
+        // them by the finer one, so the decision is the decode path's.
+        if (wave == 0) {
+#pragma unroll
+            for (int m = 0; m < NS; ++m) {
+                const uint32_t e = lane + 64u * m;
+                if (e < E) {
+                    s_S[e] = rd.S[m];
+                    s_B[e] = rd.B[m];
+                    if (!(rd.S[m] + rd.B[m] < w.lo_min_sel)) s_cand[atomicAdd(&s_ncand, 1u)] = e;
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t nc = s_ncand;
+        for (uint32_t c = wave; c < nc; c += 4u) {
+            const uint32_t e = s_cand[c];
+            double S, B;
+            router_row_sum_bound(a.router + static_cast<uint64_t>(e) * a.hidden, xs, a.hidden / 256u, S, B);
+            if (lane == 0u) {
+                s_S[e] = S;
+                s_B[e] = B;
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int m = 0; m < NS; ++m) {
+                const uint32_t e = lane + 64u * m;
+                rd.S[m] = s_S[e < E ? e : 0u];
+                rd.B[m] = s_B[e < E ? e : 0u];
+            }
+            rank();
+        }
+        __syncthreads();
+        state = s_state;
+    }
     if (state == 2u) {
         if (wave == 0) flag_router_error(a);
         return;
     }
     uint32_t sel[kMaxTopK];
     if (state == 1u) {  // rare: exact serial logits of the candidates
-        exact_routes<4, 256>(a, s_lo, xs, fb, true);
+        exact_routes<4, 256>(a, s_S, s_B, s_lo, xs, fb, true);
         if (fb.bad) {
             if (wave == 0) flag_router_error(a);
             return;
@@ -390,18 +546,13 @@ bool moe_prefill_supported(uint32_t gate_type, uint32_t up_type, uint32_t down_t
 hipError_t launch_prefill_routing(const MoePrefillArgs& a, hipStream_t s) {
     const MoeDecodeArgs& L = a.layer;
     // 1. router
-    const uint32_t per = L.hidden / kRouterThreads;
-    const uint32_t rw = per <= 8u ? 4u : per <= 16u ? 2u : 1u;  // router_rows_per_wave<per>()
-    const dim3 rgrid(ceil_div_u(L.n_experts + L.variant, 4u * rw), ceil_div_u(a.tokens, kRouterTokens));
-    switch (L.hidden / kRouterThreads) {
-#define PK_RB(C)                                                                              \
-    case C:                                                                                   \
-        hipLaunchKernelGGL(k_router_batch<C>, rgrid, dim3(kRouterThreads), 0, s, a);           \
-        break;
-        PK_RB(2) PK_RB(4) PK_RB(8) PK_RB(12) PK_RB(16) PK_RB(24) PK_RB(32)
-#undef PK_RB
-        default: return hipErrorInvalidValue;
-    }
+    const uint32_t ER = L.n_experts + L.variant;
+    if (ceil_div_u(ER, 32u) * ceil_div_u(a.tokens, 16u) >= kGemmSlots)
+        hipLaunchKernelGGL((k_router_batch<2, 4>), dim3(ceil_div_u(ER, 32u), ceil_div_u(a.tokens, 16u)),
+                           dim3(64 * kRtWaves), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_router_batch<1, 2>), dim3(ceil_div_u(ER, 16u), ceil_div_u(a.tokens, 8u)),
+                           dim3(64 * kRtWaves), 0, s, a);
     // 2. ranking
     const size_t xlds = L.hidden * sizeof(float);
     switch (slots_for(L.n_experts)) {

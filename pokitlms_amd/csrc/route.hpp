@@ -401,8 +401,9 @@ struct FallbackShared {
 // The decode gate/up kernel stages 128-value chunks (its LDS and register
 // budget), the prefill ranking kernel 256-value chunks (half the barriers).
 template <uint32_t D, uint32_t CH>
-__device__ __forceinline__ void exact_routes(const MoeDecodeArgs& a, double lo_min_sel,
-                                             const float* xs, FallbackShared<CH>& fb, bool count) {
+__device__ __forceinline__ void exact_routes(const MoeDecodeArgs& a, const double* S, const double* B,
+                                             double lo_min_sel, const float* xs, FallbackShared<CH>& fb,
+                                             bool count) {
     constexpr uint32_t PP = kStageRows * CH / 4u / 256u;  // float4 pieces per thread and chunk
     constexpr uint32_t SS = CH + 4u;
     static_assert(PP * 256u * 4u == kStageRows * CH, "whole pieces per thread of 256");
@@ -413,7 +414,7 @@ __device__ __forceinline__ void exact_routes(const MoeDecodeArgs& a, double lo_m
     }
     __syncthreads();
     if (t < E) {
-        const double s = a.row_sum[t], b = a.row_bound[t];
+        const double s = S[t], b = B[t];
         // An expert with hi < lo_min_sel is below k certain experts; every other
         // expert gets its exact CPU logit.  FP32 rounding of S keeps the rest
         // below lo_min_sel (|fl(S) - S| <= u|S| <= bound).
@@ -601,6 +602,17 @@ __device__ __forceinline__ void router_lane_sums(const rf32x4 (&w)[N4], const rf
     for (int k = 0; k < RouterLane<N4>::K; ++k) router_chunk_sums(&w[2 * k], &x[2 * k], r.local[k], r.run_abs[k]);
 }
 
+template <int N>
+struct Pieces { static constexpr int n = N; };
+
+// B from q >= sum_i |T_i|.  u = 2^-24; (1 + 2^-10) >= 1/(1 - n u) for n <= 2^13 and
+// covers the FP64 rounding of the prefix sums; q * 2^-39 >= sum |p| * 2^-40
+// covers S.
+__device__ __forceinline__ double router_bound(double q) {
+    const double b = q * (0x1p-24 * (1.0 + 0x1p-10) + 0x1p-39);
+    return q < 5.0e35 ? b : INFINITY;  // near FP32 overflow: always recompute
+}
+
 // S and B of the row whose chunk sums the wave holds (uniform results).
 //
 // S: the FP64 sum of the products (chunk sums in chunk order within a lane,
@@ -610,8 +622,9 @@ __device__ __forceinline__ void router_lane_sums(const rf32x4 (&w)[N4], const rf
 // chunk's offset (every earlier product) and L_i its own running sum,
 // sum_i |O + L_i| <= 8 |O| + sum_i |L_i| (about 8% above the exact prefixes
 // on router-like rows of 2,048).  sum_i |p_i| <= 2 sum_i |T_i| covers the FP64
-// rounding of S.  The batched prefill router calls the same functions, so
-// both paths rank on the same bits.
+// rounding of S.  The batched prefill router certifies with a coarser bound
+// first and calls the same functions for what that leaves open, so both paths make
+// the same decisions.
 template <int N4>
 __device__ __forceinline__ void router_wave_sum_bound(const RouterLane<N4>& r, double& total,
                                                       double& bound) {
@@ -627,11 +640,49 @@ __device__ __forceinline__ void router_wave_sum_bound(const RouterLane<N4>& r, d
         qs += __builtin_fma(8.0, fabs(off), r.run_abs[k]);
         off += r.local[k];
     }
-    const double q = lane63(group_sum<64>(qs));
-    // u = 2^-24; (1 + 2^-10) >= 1/(1 - n u) for n <= 2^13 and covers the FP64
-    // rounding of the prefix sums; q * 2^-39 >= sum |p| * 2^-40 covers S
-    bound = q * (0x1p-24 * (1.0 + 0x1p-10) + 0x1p-39);
-    if (!(q < 5.0e35)) bound = INFINITY;  // near FP32 overflow: always recompute
+    bound = router_bound(lane63(group_sum<64>(qs)));
+}
+
+// router_lane_sums and router_wave_sum_bound of one row with the number of
+// float4 pieces per lane known at run time (x in LDS): the same sums in the same
+// order, so the same bits.
+__device__ __forceinline__ void router_row_sum_bound(const float* row, const float* xs, uint32_t n4,
+                                                     double& total, double& bound) {
+    const uint32_t lane = threadIdx.x & 63u;
+    auto fixed = [&](auto pieces) {
+        constexpr int N4 = decltype(pieces)::n;
+        rf32x4 w[N4], x[N4];
+        router_lane_load<N4>(row, lane, w);
+        router_lane_load<N4>(xs, lane, x);
+        RouterLane<N4> r;
+        router_lane_sums<N4>(w, x, r);
+        router_wave_sum_bound<N4>(r, total, bound);
+    };
+    if (n4 == 2u) return fixed(Pieces<2>{});
+    if (n4 == 4u) return fixed(Pieces<4>{});
+    if (n4 == 8u) return fixed(Pieces<8>{});
+    // wider rows: the chunk sums formed twice instead of held
+    const rf32x4* w = reinterpret_cast<const rf32x4*>(row) + lane * n4;
+    const rf32x4* x = reinterpret_cast<const rf32x4*>(xs) + lane * n4;
+    auto chunk = [&](uint32_t k, double& l, double& ra) {
+        const rf32x4 wv[2] = {w[2u * k], w[2u * k + 1u]}, xv[2] = {x[2u * k], x[2u * k + 1u]};
+        router_chunk_sums(wv, xv, l, ra);
+    };
+    double lane_sum, l, ra;
+    chunk(0u, lane_sum, ra);
+    for (uint32_t k = 1; k < n4 / 2u; ++k) {
+        chunk(k, l, ra);
+        lane_sum += l;
+    }
+    const double incl = wave_inclusive_scan(lane_sum);
+    total = lane63(incl);
+    double off = incl - lane_sum, qs = 0.0;
+    for (uint32_t k = 0; k < n4 / 2u; ++k) {
+        chunk(k, l, ra);
+        qs += __builtin_fma(8.0, fabs(off), ra);
+        off += l;
+    }
+    bound = router_bound(lane63(group_sum<64>(qs)));
 }
 
 // Marks a router error (wave 0 of gate/up workgroup 0): route_experts throws
