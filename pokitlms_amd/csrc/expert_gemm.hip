@@ -67,14 +67,18 @@ __device__ __forceinline__ uint32_t pk_mul_f16(uint32_t a, f16x2 b) {
 // integer below 2^11, whose bits are the fp16 value 2^-24 times it (subnormals
 // and the first binade are linear), so a masked pair times the scale pair
 // (v_pk_mul_lo_u16) is the operand and only d and the mins are left outside.
-//  * Q4_K (kUnits): the accumulator is kept in units of the superblock's d and
+//  * Q4_K in the MoE block (kUnits): the accumulator is kept in units of the superblock's d and
 //    rescaled by d_prev / d once per 256 values.  The mins' term is one more
 //    MFMA per superblock: the eight integer mins against the eight group sums of
 //    x (split hi and lo, 16 operand values).
-//  * Q5_K: q - 16 and a partial sum per superblock, the rest of the mins' term
-//    (16 d sc - dmin m) times the FP32 group sums on FP32 MFMA; as Q4_K it had
-//    6.1e-7 against the 3.6e-7 of the kernel before it (the larger quants
-//    leave more to cancel against the mins).
+//  * Q5_K, and Q4_K in the prompt's projections: q - 16 (q - 8) and a partial sum per
+//    superblock, the rest of the mins' term (16 d sc - dmin m) times the FP32 group
+//    sums on FP32 MFMA.  As kUnits, Q5_K had 6.1e-7 against the 3.6e-7 of the kernel
+//    before it (the larger quants leave more to cancel against the mins), and Q4_K
+//    projections at 8.7e-7 (4.0e-7 so) put the whole model's logits 15% further from
+//    float64, as fewer FP16 roundings of k then agree; the MoE block's gate/up keeps
+//    the units, 472 against 557 us at 4096 tokens and five times more exact than the
+//    bf16 parts before.
 //
 // The others: quants as exact fp16 integers around zero (1024 + q by or-ing the
 // exponent in, minus 1024 and the offset), and per scale group (32 values;
@@ -82,11 +86,11 @@ __device__ __forceinline__ uint32_t pk_mul_f16(uint32_t a, f16x2 b) {
 // (Small integers as subnormal codes would lose bits: the MFMA aligns them as if
 // their top bit were set.)
 
-template <int T>
+template <int T, bool UNITS>
 struct WTraits {
     static constexpr bool kSuper = T == T_Q4_K || T == T_Q5_K;
     static constexpr bool kMins = kSuper || T == T_Q4_1;
-    static constexpr bool kUnits = T == T_Q4_K;           // accumulator in units of d
+    static constexpr bool kUnits = T == T_Q4_K && UNITS;           // accumulator in units of d
     static constexpr bool kMinsF32 = kMins && !kUnits;    // mins' term on FP32 MFMA
     static constexpr bool kHalfRuns = kSuper || T == T_Q8_0;
     static constexpr uint32_t kGroup = T == T_Q6_K ? 16u : 32u;
@@ -103,7 +107,7 @@ template <> struct WRaw<T_Q4_1> { uint32_t q[4][2]; uint32_t dm[4]; };  // ring 
 // What a superblock's steps share, taken from the header fields at its start
 // (which then reload for the next superblock).
 template <int T> struct WHead;
-template <> struct WHead<T_Q4_K> { uint32_t sc[2]; };
+template <> struct WHead<T_Q4_K> { uint32_t sc[2]; float cn[4]; float d; };
 template <> struct WHead<T_Q5_K> { uint32_t sc[2]; uint32_t qh[4]; float cn[4]; float d; };
 template <> struct WHead<T_Q6_K> { uint32_t sc[4]; float d; };
 template <> struct WHead<T_Q8_0> { uint32_t d[4]; };
@@ -241,7 +245,7 @@ __device__ __forceinline__ float half_of(const uint32_t* w, uint32_t i) {
 constexpr uint32_t h16x2(uint32_t bits) { return bits | (bits << 16); }
 
 // Step j's two B fragments, and (no kSuper) the scale of each.
-template <int T>
+template <int T, bool UNITS>
 __device__ __forceinline__ void wfrag(const WRaw<T>& r, const WHead<T>& hd, uint32_t j, f16x8 (&b)[2],
                                       float (&ds)[2]) {
     uint32_t w[8];
@@ -251,7 +255,7 @@ __device__ __forceinline__ void wfrag(const WRaw<T>& r, const WHead<T>& hd, uint
         const f16x2 k4096 = {static_cast<_Float16>(4096.0f), static_cast<_Float16>(4096.0f)};
         uint32_t mid = 0u;  // set below: -16 sc 2^-12
         const uint32_t scp = __builtin_amdgcn_perm(0u, hd.sc[j / 4u], 0x0c000c00u + 0x00010001u * (j % 4u));
-        if constexpr (T == T_Q5_K) mid = pk_mul_f16((scp << 4) | 0x80008000u, k4096);
+        if constexpr (!WTraits<T, UNITS>::kUnits) mid = pk_mul_f16((scp << (T == T_Q5_K ? 4 : 3)) | 0x80008000u, k4096);
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) {
             uint32_t e, o;
@@ -267,7 +271,7 @@ __device__ __forceinline__ void wfrag(const WRaw<T>& r, const WHead<T>& hd, uint
             }
             w[2u * i] = pk_mul_u16(e, scp);
             w[2u * i + 1u] = pk_mul_u16(o, scp);
-            if constexpr (T == T_Q5_K) {  // sc (q - 16) 2^-12: normal values, exact
+            if constexpr (!WTraits<T, UNITS>::kUnits) {  // sc (q - 16) 2^-12: normal values, exact
                 w[2u * i] = pk_fma16(w[2u * i], k4096, mid);
                 w[2u * i + 1u] = pk_fma16(w[2u * i + 1u], k4096, mid);
             }
@@ -318,10 +322,10 @@ __device__ __forceinline__ void wfrag(const WRaw<T>& r, const WHead<T>& hd, uint
 // fp16 codes), the factor that brings the accumulator from the units of the
 // superblock before (dcur) to this one's, and the mins' coefficient there.  A
 // zero d keeps the units and zeroes the scales.
-template <int T>
+template <int T, bool UNITS>
 __device__ __forceinline__ void whead(const WRaw<T>& r, WHead<T>& hd, uint32_t kq, f16x8& mins,
                                       float& dcur, float& rescale, float& cmin) {
-    using W = WTraits<T>;
+    using W = WTraits<T, UNITS>;
     if constexpr (T == T_Q4_K || T == T_Q5_K) {
         const float d = half_bits_to_float(r.h[0] & 0xffffu);
         const float dmin = half_bits_to_float(r.h[0] >> 16);
@@ -332,7 +336,7 @@ __device__ __forceinline__ void whead(const WRaw<T>& r, WHead<T>& hd, uint32_t k
         hd.sc[1] = ((r.h[3] & 0x0f0f0f0fu) | ((r.h[1] >> 2) & 0x30303030u)) & keep;
         const uint32_t m0 = r.h[2] & 0x3f3f3f3fu;
         const uint32_t m1 = ((r.h[3] >> 4) & 0x0f0f0f0fu) | ((r.h[2] >> 2) & 0x30303030u);
-        if constexpr (T == T_Q4_K) {
+        if constexpr (W::kUnits) {
             mins = frag4(__builtin_amdgcn_perm(0u, m0, 0x0c010c00u) << 4,
                          __builtin_amdgcn_perm(0u, m0, 0x0c030c02u) << 4,
                          __builtin_amdgcn_perm(0u, m1, 0x0c010c00u) << 4,
@@ -345,11 +349,11 @@ __device__ __forceinline__ void whead(const WRaw<T>& r, WHead<T>& hd, uint32_t k
             hd.d = d * 0x1p12f;
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {  // 16 d sc_j - dmin m_j of group j = 2 i + kq
-                hd.qh[i] = r.qh[i];
+                if constexpr (T == T_Q5_K) hd.qh[i] = r.qh[i];
                 const uint32_t sh = 16u * (i & 1u) + 8u * kq;
                 const float m = static_cast<float>(((i < 2u ? m0 : m1) >> sh) & 0xffu);
                 const float sc = static_cast<float>((hd.sc[i / 2u] >> sh) & 0xffu);
-                hd.cn[i] = __fmaf_rn(-dmin, m, __fmul_rn(16.0f * d, sc));
+                hd.cn[i] = __fmaf_rn(-dmin, m, __fmul_rn((T == T_Q5_K ? 16.0f : 8.0f) * d, sc));
             }
         }
     } else if constexpr (T == T_Q6_K) {
@@ -418,15 +422,18 @@ __device__ __forceinline__ float half_wave_max(float v) {
 // MT x 32 assignments of a tile, from its row row0.  DUAL: gate and up rows n0 .. n0 + 127 over x,
 // SwiGLU, activations split for the down GEMM; otherwise down rows n0 .. n0 + 255
 // over the activations, each output row to its (token, route) slot.
-template <int T, bool DUAL, int MT>
+template <int T, bool UNITS, bool DUAL, int MT>
 __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef& tr, uint32_t n0,
                                           GemmShared& sh, uint32_t row0 = 0u) {
-    using W = WTraits<T>;
+    using W = WTraits<T, UNITS>;
     const MoeDecodeArgs& L = a.layer;
     const uint32_t kdim = DUAL ? L.hidden : L.ffn, ndim = DUAL ? L.ffn : L.hidden;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t ln = lane % 32u, kq = lane / 32u;
-    const uint32_t nsb = kdim / 256u, nst = kdim / 32u;
+    const uint32_t nst = kdim / 32u;
+    // superblocks sb0 .. nsb - 1 of K: all, or this workgroup's share (dense GEMMs)
+    const uint32_t all = kdim / 256u, parts_k = DUAL ? 1u : a.k_parts;
+    const uint32_t sb0 = blockIdx.y * all / parts_k, nsb = (blockIdx.y + 1u) * all / parts_k;
 
     // weights
     const bool shared = tr.e >= L.n_experts;  // the shared expert (variant 1): its own tensors
@@ -446,9 +453,9 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     WRaw<T> raw[2];
 #pragma unroll
     for (uint32_t i = 0; i < 2; ++i) {
-        wload_head<T>(ws[i], blk, 0u, kq, raw[i]);
+        wload_head<T>(ws[i], blk, sb0, kq, raw[i]);
 #pragma unroll
-        for (uint32_t j = 0; j < (T == T_Q8_0 || T == T_Q4_1 ? 4u : 8u); ++j) wload_step<T>(ws[i], blk, 0u, j, kq, raw[i]);
+        for (uint32_t j = 0; j < (T == T_Q8_0 || T == T_Q4_1 ? 4u : 8u); ++j) wload_step<T>(ws[i], blk, sb0, j, kq, raw[i]);
     }
 
     // activations: thread t moves piece t % 8 (16 bytes) of rows t / 8 (+ 32)
@@ -473,7 +480,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     constexpr uint32_t NS = MT == 1 ? 8u : 2u;
     u32x4_t av[NS][MT];
     float ac[NS][MT];
-    const uint32_t last = nst - 1u;
+    const uint32_t last = 8u * nsb - 1u;
     auto load_act = [&](uint32_t set, uint32_t s) {  // past the end: the last stage again
         const uint32_t st = s < last ? s : last;
 #pragma unroll
@@ -528,13 +535,13 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
                                              sh.xs[buf] + (ln + 32u * m) * 32u + kq * 16u));
     };
 
-    load_act(0u, 0u);
-    load_sums(0u);
+    load_act(0u, 8u * sb0);
+    load_sums(sb0);
 #pragma unroll
-    for (uint32_t i = 1; i < NS; ++i) load_act(i, i);
+    for (uint32_t i = 1; i < NS; ++i) load_act(i, 8u * sb0 + i);
     store_act(0u, 0u);
-    store_sums(0u);
-    load_act(0u, NS);
+    store_sums(sb0 & 1u);
+    load_act(0u, 8u * sb0 + NS);
     __syncthreads();
 
     f32x16 acc[MT][2], part[MT][2];  // part: Q5_K, the superblock's sums
@@ -542,14 +549,14 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = f32x16{};
     float dcur[2] = {1.0f, 1.0f};
     WHead<T> hd[2];
-    for (uint32_t sb = 0; sb < nsb; ++sb) {
+    for (uint32_t sb = sb0; sb < nsb; ++sb) {
         const uint32_t bn = sb + 1u < nsb ? sb + 1u : nsb - 1u, sbuf = sb & 1u;
         {
             f16x8 mins[2];
             float rescale[2], cmin[2];
 #pragma unroll
             for (uint32_t i = 0; i < 2; ++i) {
-                whead<T>(raw[i], hd[i], kq, mins[i], dcur[i], rescale[i], cmin[i]);
+                whead<T, UNITS>(raw[i], hd[i], kq, mins[i], dcur[i], rescale[i], cmin[i]);
                 wload_head<T>(ws[i], blk, bn, kq, raw[i]);
             }
             if constexpr (W::kUnits) {
@@ -573,7 +580,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
             f16x8 b[2][2];
             float ds[2][2];
 #pragma unroll
-            for (uint32_t i = 0; i < 2; ++i) wfrag<T>(raw[i], hd[i], j, b[i], ds[i]);
+            for (uint32_t i = 0; i < 2; ++i) wfrag<T, UNITS>(raw[i], hd[i], j, b[i], ds[i]);
             if constexpr (T == T_Q4_1) {  // the mins of groups 2 i + kq
 #pragma unroll
                 for (uint32_t i = 0; i < 2; ++i) {
@@ -693,6 +700,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
             }
         }
     } else {
+        float* out = a.out + blockIdx.y * a.out_part;
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -700,7 +708,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
                 const uint32_t row = row0 + 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
                 if (row < tr.rows) {
                     const float s = sh.scale[row];
-                    float* o = a.out + static_cast<uint64_t>(sh.oslot[row]) * ndim + n0 + wave * 32u + ln;
+                    float* o = out + static_cast<uint64_t>(sh.oslot[row]) * ndim + n0 + wave * 32u + ln;
                     o[0] = acc[m][0][r] * u0 * s;
                     o[kRowsN] = acc[m][1][r] * u1 * s;
                 }
@@ -708,7 +716,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     }
 }
 
-template <int T, bool DUAL>
+template <int T, bool UNITS, bool DUAL>
 __global__ __launch_bounds__(256, 2) void k_expert_gemm(MoePrefillArgs a) {
     __shared__ __attribute__((aligned(16))) GemmShared sh;
     const MoeDecodeArgs& L = a.layer;
@@ -741,12 +749,12 @@ __global__ __launch_bounds__(256, 2) void k_expert_gemm(MoePrefillArgs a) {
     if constexpr (T == T_Q4_1) {  // its scales and mins leave no registers for two row blocks
         for (uint32_t row0 = 0; row0 < tr.rows; row0 += 32u) {
             if (row0) __syncthreads();
-            gemm_tile<T, DUAL, 1>(a, tr, yb * nblk, sh, row0);
+            gemm_tile<T, UNITS, DUAL, 1>(a, tr, yb * nblk, sh, row0);
         }
     } else if (tr.rows > 32u) {
-        gemm_tile<T, DUAL, 2>(a, tr, yb * nblk, sh);
+        gemm_tile<T, UNITS, DUAL, 2>(a, tr, yb * nblk, sh);
     } else {
-        gemm_tile<T, DUAL, 1>(a, tr, yb * nblk, sh);
+        gemm_tile<T, UNITS, DUAL, 1>(a, tr, yb * nblk, sh);
     }
 }
 
@@ -755,7 +763,14 @@ hipError_t expert_gemm_t(const MoePrefillArgs& a, hipStream_t s) {
     const MoeDecodeArgs& L = a.layer;
     const uint32_t nb = DUAL ? L.ffn / kRowsN : L.hidden / (2u * kRowsN);
     const uint32_t blocks = 8u * ((a.max_tiles + 7u) / 8u) * nb;  // xcd_tile's layout
-    hipLaunchKernelGGL((k_expert_gemm<T, DUAL>), dim3(blocks), dim3(256), 0, s, a);
+    const dim3 grid(blocks, DUAL ? 1u : a.k_parts);
+    if constexpr (T == T_Q4_K && !DUAL) {
+        if (a.precise) {
+            hipLaunchKernelGGL((k_expert_gemm<T, false, DUAL>), grid, dim3(256), 0, s, a);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((k_expert_gemm<T, T == T_Q4_K, DUAL>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -133,6 +133,10 @@ struct MoePrefillArgs {
     float* act_scale;        // [P][ffn / 32]: each stage's scale
     float* out;              // [P][hidden], slot token * top_k + route
     uint32_t* status;        // as MoeDecodeArgs::status
+    // down GEMM only: K split over k_parts workgroups, part p's sums at out + p * out_part
+    uint32_t k_parts = 1;
+    uint32_t precise = 0;    // Q4_K: partial sums per superblock of quants around zero
+    uint64_t out_part = 0;
 };
 uint32_t moe_prefill_tile_wgs(uint32_t hidden, uint32_t ffn);
 uint32_t moe_prefill_max_tiles(uint32_t tokens, uint32_t top_k, uint32_t n_experts);
@@ -213,6 +217,35 @@ hipError_t launch_fast_add_rmsnorm(float* x, const float* d, const float* w, flo
 // logits: run the final norm, head and argmax (else only advance the position).
 hipError_t launch_model_step(const ModelArgs& a, const ModelLayer* layers, bool logits,
                              hipStream_t stream);
+
+// The fast mode's prompt in batches (prompt.hip).
+constexpr uint32_t kPromptTokens = 512;  // positions per chunk
+struct PromptArgs {
+    ModelArgs m;
+    MoePrefillArgs moe;       // the MoE blocks' scratch
+    uint32_t tokens, dense_tiles, moe_tiles;
+    float *h, *x, *y;         // [tokens][hidden]: residual stream, normed, MoE output
+    float* qr;                // [tokens][heads * head_dim]: q after norm and RoPE
+    float* proj;              // the projections' parts
+    float* attn_out;          // the output projection's parts [part][tokens][hidden]
+    uint16_t* op_parts;       // the dense GEMMs' operand (gemm_split.hpp, a scale per stage)
+    float *op_scale, *op_sums;
+    uint32_t *d_tiles, *d_offsets, *d_perm;
+    // per layer: where q, k and v of position t are (row stride, stride of the K parts)
+    const float *q, *k, *v;
+    uint32_t q_stride, kv_stride, qkv_parts;
+    uint64_t q_part, kv_part;
+};
+bool prompt_supported(const ModelArgs& m, const ModelLayer* layers);
+// Carves the scratch for chunks of up to `tokens` out of base (null: only the size).
+uint64_t prompt_scratch(const ModelArgs& m, const ModelLayer* layers, uint32_t tokens, uint8_t* base,
+                        PromptArgs& a);
+// Positions pos0 .. pos0 + tokens - 1 (state[0] = pos0, pos0 + tokens <= capacity)
+// through every layer, into the KV ring; advances state[0].
+hipError_t launch_prompt_chunk(PromptArgs a, const ModelLayer* layers, uint32_t tokens, uint32_t pos0,
+                               hipStream_t stream);
+// Embedding rows of tokens[state[0] + i], i < rows, into hidden_state rows.
+hipError_t launch_embed(const ModelArgs& a, uint32_t rows, hipStream_t stream);
 
 // Rows [first_row, first_row + rows) of a slice (rows_in_slice rows of `in`
 // elements) as FP32, decoded exactly as the embedding row (every type the
