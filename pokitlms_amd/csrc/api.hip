@@ -1375,6 +1375,10 @@ struct pk_hip_qwen3moe {
     uint8_t* prompt_mem = nullptr;
     uint32_t prompt_tokens = 0;
     pk::PromptArgs prompt{};
+    // reference order: per position of a chunk, the step's buffers
+    uint64_t ref_tok = 0;
+    uint32_t* ref_ids = nullptr;
+    float* ref_probs = nullptr;
     hipGraphExec_t step_logits = nullptr, step_plain = nullptr;
     hipEvent_t ev[2] = {};
 };
@@ -1446,13 +1450,15 @@ void release_model(pk_hip_qwen3moe* m) {
 // positions: 319 against 336 us for one layer, 698 against 667 for three; 5: 327
 // against 378, 700 against 785).
 constexpr uint32_t kPromptMin = 5;
+// The reference order's chunk costs about as much as two of its steps and 20 us per
+// position and layer more, a step 74 (2 positions: 347 against 363 us for one layer,
+// 760 against 762 for three; 3: 376 against 444, 851 against 984; 127: 3077 against
+// 10318, 8336 against 28236).
+constexpr uint32_t kRefPromptMin = 2;
 
-// Scratch for chunks of min(n, kPromptTokens) positions, kept with the model; false
-// where memory for it is short (the token steps need none).
-bool prompt_scratch_ready(pk_hip_qwen3moe* m, uint32_t n) {
-    const uint32_t t = std::min(n <= 64 ? 64u : n <= 192 ? 192u : pk::kPromptTokens, pk::kPromptTokens);
-    if (m->prompt_tokens >= t) return true;
-    const uint64_t bytes = pk::prompt_scratch(m->args, m->layers.data(), t, nullptr, m->prompt);
+// The prompt's scratch is kept with the model and given back with it.  False where
+// memory for it is short (the token steps need none).
+bool grow_prompt_mem(pk_hip_qwen3moe* m, uint64_t bytes, uint32_t tokens) {
     uint8_t* mem = nullptr;
     if (hipMalloc(&mem, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -1460,8 +1466,50 @@ bool prompt_scratch_ready(pk_hip_qwen3moe* m, uint32_t n) {
     }
     if (m->prompt_mem) (void)hipFree(m->prompt_mem);
     m->prompt_mem = mem;
-    m->prompt_tokens = t;
-    pk::prompt_scratch(m->args, m->layers.data(), t, mem, m->prompt);
+    m->prompt_tokens = tokens;
+    return true;
+}
+
+// Fast mode: scratch for chunks of min(n, kPromptTokens) positions.
+bool prompt_scratch_ready(pk_hip_qwen3moe* m, uint32_t n) {
+    const uint32_t t = std::min(n <= 64 ? 64u : n <= 192 ? 192u : pk::kPromptTokens, pk::kPromptTokens);
+    if (m->prompt_tokens >= t) return true;
+    const uint64_t bytes = pk::prompt_scratch(m->args, m->layers.data(), t, nullptr, m->prompt);
+    if (!grow_prompt_mem(m, bytes, t)) return false;
+    pk::prompt_scratch(m->args, m->layers.data(), t, m->prompt_mem, m->prompt);
+    return true;
+}
+
+// Reference order: each position's copy of the step's buffers, 256-byte aligned.
+bool ref_prompt_ready(pk_hip_qwen3moe* m, uint32_t n, pk::ModelArgs& a) {
+    const uint64_t H = a.hidden, qd = uint64_t(a.heads) * a.head_dim, kd = uint64_t(a.kv_heads) * a.head_dim;
+    uint64_t ffn = 1;
+    for (const pk::ModelLayer& L : m->layers) ffn = std::max<uint64_t>(ffn, L.moe.ffn);
+    uint64_t at = 0;
+    auto take = [&](uint64_t words) {
+        const uint64_t here = at;
+        at += (words + 63) / 64 * 64;
+        return here;
+    };
+    const uint64_t hidden = take(H), alt = take(H), normed = take(H), attn = take(H), q = take(qd),
+                   k = take(kd), v = take(kd), att = take(qd),
+                   scratch = take(pk::ref_scratch_floats(m->cfg.top_k, static_cast<uint32_t>(ffn), a.hidden)),
+                   ids = take(16), probs = take(16);
+    const uint32_t t = std::min(n <= 32 ? 32u : pk::kRefPromptTokens, pk::kRefPromptTokens);
+    if (m->prompt_tokens < t && !grow_prompt_mem(m, at * t * sizeof(float), t)) return false;
+    float* p = reinterpret_cast<float*>(m->prompt_mem);
+    m->ref_tok = at;
+    m->ref_ids = reinterpret_cast<uint32_t*>(p + ids);
+    m->ref_probs = p + probs;
+    a.hidden_state = p + hidden;
+    a.hidden_alt = p + alt;
+    a.normed = p + normed;
+    a.attn_out = p + attn;
+    a.q = p + q;
+    a.k = p + k;
+    a.v = p + v;
+    a.att = p + att;
+    a.ref_scratch = p + scratch;
     return true;
 }
 
@@ -1721,8 +1769,15 @@ pk_hip_status pk_hip_qwen3moe_generate(pk_hip_qwen3moe* m, const uint32_t* promp
         uint32_t done = 0;
         // all but the last prompt token that the KV window holds, in chunks
         const uint32_t batch = std::min(n_prompt - 1, m->cfg.kv_capacity);
-        if (batch >= kPromptMin && pk::prompt_supported(m->args, m->layers.data()) &&
-            prompt_scratch_ready(m, batch)) {
+        pk::ModelArgs chunk = m->args;
+        if (batch >= kRefPromptMin && pk::ref_prompt_supported(m->args, m->layers.data()) &&
+            ref_prompt_ready(m, batch, chunk)) {
+            for (; done < batch; done += std::min(batch - done, m->prompt_tokens))
+                check(pk::launch_ref_prompt_chunk(chunk, m->layers.data(), m->ref_ids, m->ref_probs,
+                                                  std::min(batch - done, m->prompt_tokens), m->ref_tok, s),
+                      "prompt chunk");
+        } else if (batch >= kPromptMin && pk::prompt_supported(m->args, m->layers.data()) &&
+                   prompt_scratch_ready(m, batch)) {
             m->prompt.m = m->args;
             for (; done < batch; done += std::min(batch - done, m->prompt_tokens))
                 check(pk::launch_prompt_chunk(m->prompt, m->layers.data(),

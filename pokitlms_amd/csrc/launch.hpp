@@ -218,6 +218,15 @@ hipError_t launch_fast_add_rmsnorm(float* x, const float* d, const float* w, flo
 hipError_t launch_model_step(const ModelArgs& a, const ModelLayer* layers, bool logits,
                              hipStream_t stream);
 
+// The reference order's prompt in batches: positions pos0 .. of a chunk (state[0] =
+// pos0, all inside the KV window) through every layer, position t's buffers (those
+// a points to, and ids / probs) t * tok words after position 0's; advances state[0].
+constexpr uint32_t kRefPromptTokens = 128;  // positions per chunk
+bool ref_prompt_supported(const ModelArgs& a, const ModelLayer* layers);
+hipError_t launch_ref_prompt_chunk(const ModelArgs& a, const ModelLayer* layers, uint32_t* ids,
+                                   float* probs, uint32_t tokens, uint64_t tok, hipStream_t stream);
+hipError_t launch_advance(uint32_t* state, uint32_t n, hipStream_t stream);
+
 // The fast mode's prompt in batches (prompt.hip).
 constexpr uint32_t kPromptTokens = 512;  // positions per chunk
 struct PromptArgs {
@@ -244,8 +253,8 @@ uint64_t prompt_scratch(const ModelArgs& m, const ModelLayer* layers, uint32_t t
 // through every layer, into the KV ring; advances state[0].
 hipError_t launch_prompt_chunk(PromptArgs a, const ModelLayer* layers, uint32_t tokens, uint32_t pos0,
                                hipStream_t stream);
-// Embedding rows of tokens[state[0] + i], i < rows, into hidden_state rows.
-hipError_t launch_embed(const ModelArgs& a, uint32_t rows, hipStream_t stream);
+// Embedding rows of tokens[state[0] + i], i < rows, into hidden_state + i * stride.
+hipError_t launch_embed(const ModelArgs& a, uint32_t rows, uint64_t stride, hipStream_t stream);
 
 // Rows [first_row, first_row + rows) of a slice (rows_in_slice rows of `in`
 // elements) as FP32, decoded exactly as the embedding row (every type the
@@ -326,6 +335,10 @@ struct RefMatvecArgs {
     LibmExpf expf;
     RefNormIn norm;           // norm.w set: x is RMSNorm(norm.x + norm.res) * norm.w
     RefRouteIn route;         // route.logits set: the expert slices come from routing
+    // the same for `tokens` positions (grid z): x, y, ids and act of position t are
+    // t * tok words on; no norm, routing or x_up then
+    uint32_t tokens = 1;
+    uint64_t tok = 0;
 };
 bool ref_matvec_supported(uint32_t type, uint32_t in);
 hipError_t launch_ref_matvec(uint32_t type, const RefMatvecArgs& a, uint32_t routes,

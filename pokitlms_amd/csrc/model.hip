@@ -215,11 +215,11 @@ __device__ void decode32(const QRow& row, uint32_t k0, float* v) {
 }
 
 // Step start: hidden = embedding row of tokens[pos] (block b: of tokens[pos + b],
-// into row b).
+// stride floats after block 0's).
 template <int T>
-__global__ __launch_bounds__(256) void k_embed(ModelArgs a) {
+__global__ __launch_bounds__(256) void k_embed(ModelArgs a, uint64_t stride) {
     const uint32_t pos = a.state[0] + blockIdx.x;
-    a.hidden_state += static_cast<uint64_t>(blockIdx.x) * a.hidden;
+    a.hidden_state += blockIdx.x * stride;
     const uint32_t token = a.tokens[pos];
     const uint32_t tid = threadIdx.x;
     // blocks per row (one element per block for the float types)
@@ -400,8 +400,8 @@ hipError_t launch_argmax(const ModelArgs& a, hipStream_t s) {
 }
 
 template <int T>
-hipError_t embed_t(const ModelArgs& a, uint32_t rows, hipStream_t s) {
-    hipLaunchKernelGGL(k_embed<T>, dim3(rows), dim3(256), 0, s, a);
+hipError_t embed_t(const ModelArgs& a, uint32_t rows, uint64_t stride, hipStream_t s) {
+    hipLaunchKernelGGL(k_embed<T>, dim3(rows), dim3(256), 0, s, a, stride);
     return hipGetLastError();
 }
 
@@ -516,28 +516,28 @@ hipError_t launch_fast_add_rmsnorm(float* x, const float* d, const float* w, flo
     return hipGetLastError();
 }
 
-hipError_t launch_embed(const ModelArgs& a, uint32_t rows, hipStream_t s) {
+hipError_t launch_embed(const ModelArgs& a, uint32_t rows, uint64_t stride, hipStream_t s) {
     switch (a.embd_type) {
-        case T_F32: return embed_t<T_F32>(a, rows, s);
-        case T_F16: return embed_t<T_F16>(a, rows, s);
-        case T_BF16: return embed_t<T_BF16>(a, rows, s);
-        case T_Q4_1: return embed_t<T_Q4_1>(a, rows, s);
-        case T_Q5_0: return embed_t<T_Q5_0>(a, rows, s);
-        case T_Q5_1: return embed_t<T_Q5_1>(a, rows, s);
-        case T_Q2_K: return embed_t<T_Q2_K>(a, rows, s);
-        case T_Q3_K: return embed_t<T_Q3_K>(a, rows, s);
-        case T_Q4_K: return embed_t<T_Q4_K>(a, rows, s);
-        case T_Q5_K: return embed_t<T_Q5_K>(a, rows, s);
-        case T_Q6_K: return embed_t<T_Q6_K>(a, rows, s);
-        case T_Q8_0: return embed_t<T_Q8_0>(a, rows, s);
-        case T_Q4_0: return embed_t<T_Q4_0>(a, rows, s);
+        case T_F32: return embed_t<T_F32>(a, rows, stride, s);
+        case T_F16: return embed_t<T_F16>(a, rows, stride, s);
+        case T_BF16: return embed_t<T_BF16>(a, rows, stride, s);
+        case T_Q4_1: return embed_t<T_Q4_1>(a, rows, stride, s);
+        case T_Q5_0: return embed_t<T_Q5_0>(a, rows, stride, s);
+        case T_Q5_1: return embed_t<T_Q5_1>(a, rows, stride, s);
+        case T_Q2_K: return embed_t<T_Q2_K>(a, rows, stride, s);
+        case T_Q3_K: return embed_t<T_Q3_K>(a, rows, stride, s);
+        case T_Q4_K: return embed_t<T_Q4_K>(a, rows, stride, s);
+        case T_Q5_K: return embed_t<T_Q5_K>(a, rows, stride, s);
+        case T_Q6_K: return embed_t<T_Q6_K>(a, rows, stride, s);
+        case T_Q8_0: return embed_t<T_Q8_0>(a, rows, stride, s);
+        case T_Q4_0: return embed_t<T_Q4_0>(a, rows, stride, s);
         default: return hipErrorInvalidValue;
     }
 }
 
 hipError_t launch_model_step(const ModelArgs& a, const ModelLayer* layers, bool logits,
                              hipStream_t s) {
-    hipError_t err = launch_embed(a, 1u, s);
+    hipError_t err = launch_embed(a, 1u, 0u, s);
     if (err != hipSuccess) return err;
     if (a.exact) {
         if ((err = launch_ref_step(a, layers, logits, s))) return err;

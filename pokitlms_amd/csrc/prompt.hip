@@ -367,7 +367,7 @@ hipError_t launch_prompt_chunk(PromptArgs a, const ModelLayer* layers, uint32_t 
     a.tokens = tokens;
     ModelArgs em = m;
     em.hidden_state = a.h;
-    if ((err = launch_embed(em, tokens, s))) return err;
+    if ((err = launch_embed(em, tokens, m.hidden, s))) return err;
     // the tile list of the dense GEMMs: one for both, from the wider
     const uint32_t rows = dense_rows(tokens, qd + 2u * kd > H ? qd + 2u * kd : H);
     a.dense_tiles = (tokens + rows - 1u) / rows;
@@ -436,7 +436,11 @@ hipError_t launch_prompt_chunk(PromptArgs a, const ModelLayer* layers, uint32_t 
         if ((err = launch_prefill_down(g, s))) return err;
         delta = a.y;
     }
-    hipLaunchKernelGGL(k_prompt_advance, dim3(1), dim3(64), 0, s, m.state, tokens);
+    return launch_advance(m.state, tokens, s);
+}
+
+hipError_t launch_advance(uint32_t* state, uint32_t n, hipStream_t s) {
+    hipLaunchKernelGGL(k_prompt_advance, dim3(1), dim3(64), 0, s, state, n);
     return hipGetLastError();
 }
 
