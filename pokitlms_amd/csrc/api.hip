@@ -1450,10 +1450,10 @@ void release_model(pk_hip_qwen3moe* m) {
 // positions: 319 against 336 us for one layer, 698 against 667 for three; 5: 327
 // against 378, 700 against 785).
 constexpr uint32_t kPromptMin = 5;
-// The reference order's chunk costs about as much as two of its steps and 20 us per
-// position and layer more, a step 74 (2 positions: 347 against 363 us for one layer,
-// 760 against 762 for three; 3: 376 against 444, 851 against 984; 127: 3077 against
-// 10318, 8336 against 28236).
+// The reference order's chunk costs about as much as one of its steps and 8 us per
+// position and layer more, a step 74 (2 positions: 314 against 363 us for one layer,
+// 657 against 762 for three; 3: 330 against 444, 712 against 984; 127: 1343 against
+// 10318, 3927 against 28236).
 constexpr uint32_t kRefPromptMin = 2;
 
 // The prompt's scratch is kept with the model and given back with it.  False where

@@ -330,23 +330,36 @@ __device__ __forceinline__ uint32_t zero_after(float v) {
     return z;
 }
 
+__device__ __forceinline__ float at4(const float4& v, uint32_t i) {
+    return i == 0u ? v.x : i == 1u ? v.y : i == 2u ? v.z : v.w;
+}
+
 // dot of a loaded block with x (x in LDS, 16-byte aligned), in element
 // order.  K-quants and Q4_1: the decoded FP32 weight times x; Q8_0/Q4_0:
-// d * dot_i8_f32 (the int8 value times x, then the scale once).
-template <int T>
-__device__ float ref_dot(const RefRaw<T>& r, const float* x) {
-    const float4* x4 = reinterpret_cast<const float4*>(x);
-    float s = 0.0f;
+// d * dot_i8_f32 (the int8 value times x, then the scale once).  N inputs, xs
+// floats apart, share the decoded weights; each has its own chain.
+template <int T, int N>
+__device__ __forceinline__ void ref_dots(const RefRaw<T>& r, const float* x, uint32_t xs, float (&s)[N]) {
+    const float4* x4[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        x4[n] = reinterpret_cast<const float4*>(x + n * xs);
+        s[n] = 0.0f;
+    }
     if constexpr (T == T_Q4_K || T == T_Q5_K) {
         constexpr int QS = T == T_Q4_K ? 4 : 12;
         const uint32_t* w = r.w;
         const uint32_t h[4] = {w[0], w[1], w[2], w[3]};
         const float d = half_bits_to_float(w[0] & 0xffffu), dmin = half_bits_to_float(w[0] >> 16);
-        X8 xa = ldx8(x4, 0u);
+        X8 xa[N], xb[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n) xa[n] = ldx8(x4[n], 0u);
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) {
-            X8 xb;
-            if (j < 7u) xb = ldx8(x4 + zero_after(s), 8u * (j + 1u));
+            if (j < 7u) {
+#pragma unroll
+                for (int n = 0; n < N; ++n) xb[n] = ldx8(x4[n] + zero_after(s[n]), 8u * (j + 1u));
+            }
             float sc, mn;
             kq_scale_min(h, j, sc, mn);
             const float ds = __fmul_rn(d, sc), dm = __fmul_rn(dmin, mn);
@@ -355,17 +368,25 @@ __device__ float ref_dot(const RefRaw<T>& r, const float* x) {
                 const uint32_t raw = w[QS + 8u * (j / 2u) + k];
                 uint32_t v = (j & 1u) ? (raw >> 4) & 0x0f0f0f0fu : raw & 0x0f0f0f0fu;
                 if constexpr (T == T_Q5_K) v |= ((w[4u + k] >> j) & 0x01010101u) << 4;
-                s = kq_step4(s, ds, dm, v, xa.v[k]);
+#pragma unroll
+                for (int n = 0; n < N; ++n) s[n] = kq_step4(s[n], ds, dm, v, xa[n].v[k]);
             }
-            if (j < 7u) xa = xb;
+            if (j < 7u) {
+#pragma unroll
+                for (int n = 0; n < N; ++n) xa[n] = xb[n];
+            }
         }
     } else if constexpr (T == T_Q6_K) {
         const float d = r.d;
-        X8 xa = ldx8(x4, 0u);
+        X8 xa[N], xb[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n) xa[n] = ldx8(x4[n], 0u);
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
-            X8 xb;
-            if (c < 7u) xb = ldx8(x4 + zero_after(s), 8u * (c + 1u));
+            if (c < 7u) {
+#pragma unroll
+                for (int n = 0; n < N; ++n) xb[n] = ldx8(x4[n] + zero_after(s[n]), 8u * (c + 1u));
+            }
             const uint32_t half = c / 4u, g = c % 4u;
 #pragma unroll
             for (uint32_t k = 0; k < 8; ++k) {
@@ -376,22 +397,30 @@ __device__ float ref_dot(const RefRaw<T>& r, const float* x) {
                 const uint32_t hw = r.qh[8u * half + k];
                 const uint32_t v = (g >= 2u ? (lw >> 4) & 0x0f0f0f0fu : lw & 0x0f0f0f0fu) |
                                    (((hw >> (2u * g)) & 0x03030303u) << 4);
-                s = q6_step4(s, dsc, v, xa.v[k]);
+#pragma unroll
+                for (int n = 0; n < N; ++n) s[n] = q6_step4(s[n], dsc, v, xa[n].v[k]);
             }
-            if (c < 7u) xa = xb;
+            if (c < 7u) {
+#pragma unroll
+                for (int n = 0; n < N; ++n) xa[n] = xb[n];
+            }
         }
     } else if constexpr (T == T_Q8_0) {
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
-            const float4 xv = x4[k];
-            const float xs[4] = {xv.x, xv.y, xv.z, xv.w};
+            float4 xv[N];
+#pragma unroll
+            for (int n = 0; n < N; ++n) xv[n] = x4[n][k];
 #pragma unroll
             for (uint32_t m = 0; m < 4; ++m) {
                 const int q = static_cast<int8_t>(r.w[k] >> (8u * m));
-                s = __fadd_rn(s, __fmul_rn(xs[m], static_cast<float>(q)));
+#pragma unroll
+                for (int n = 0; n < N; ++n)
+                    s[n] = __fadd_rn(s[n], __fmul_rn(at4(xv[n], m), static_cast<float>(q)));
             }
         }
-        s = __fmul_rn(r.d, s);
+#pragma unroll
+        for (int n = 0; n < N; ++n) s[n] = __fmul_rn(r.d, s[n]);
     } else if constexpr (T == T_Q4_1) {  // weight fl(fl(q * d) + m), low nibbles first
         const uint32_t* w = r.w;         // d | m << 16, then quants 0..15
         const float d = half_bits_to_float(w[0] & 0xffffu), m = half_bits_to_float(w[0] >> 16);
@@ -399,11 +428,14 @@ __device__ float ref_dot(const RefRaw<T>& r, const float* x) {
         for (uint32_t k = 0; k < 8; ++k) {
             const uint32_t raw = w[1u + (k & 3u)];
             const uint32_t v = k < 4u ? raw & 0x0f0f0f0fu : (raw >> 4) & 0x0f0f0f0fu;
-            const float4 xv = x4[k];
-            s = __fadd_rn(s, __fmul_rn(__fadd_rn(__fmul_rn(ub<0>(v), d), m), xv.x));
-            s = __fadd_rn(s, __fmul_rn(__fadd_rn(__fmul_rn(ub<1>(v), d), m), xv.y));
-            s = __fadd_rn(s, __fmul_rn(__fadd_rn(__fmul_rn(ub<2>(v), d), m), xv.z));
-            s = __fadd_rn(s, __fmul_rn(__fadd_rn(__fmul_rn(ub<3>(v), d), m), xv.w));
+#pragma unroll
+            for (int n = 0; n < N; ++n) {
+                const float4 xv = x4[n][k];
+                s[n] = __fadd_rn(s[n], __fmul_rn(__fadd_rn(__fmul_rn(ub<0>(v), d), m), xv.x));
+                s[n] = __fadd_rn(s[n], __fmul_rn(__fadd_rn(__fmul_rn(ub<1>(v), d), m), xv.y));
+                s[n] = __fadd_rn(s[n], __fmul_rn(__fadd_rn(__fmul_rn(ub<2>(v), d), m), xv.z));
+                s[n] = __fadd_rn(s[n], __fmul_rn(__fadd_rn(__fmul_rn(ub<3>(v), d), m), xv.w));
+            }
         }
     } else if constexpr (T == T_Q5_0 || T == T_Q5_1) {
         // decode_q5_0: fl((q - 16) * d); decode_q5_1: fl(fl(q * d) + m)
@@ -424,8 +456,9 @@ __device__ float ref_dot(const RefRaw<T>& r, const float* x) {
         }
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
-            const float4 xv = x4[k];
-            const float xs[4] = {xv.x, xv.y, xv.z, xv.w};
+            float4 xv[N];
+#pragma unroll
+            for (int n = 0; n < N; ++n) xv[n] = x4[n][k];
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j) {
                 const uint32_t i = 4u * k + j, byte = i & 15u;
@@ -433,7 +466,8 @@ __device__ float ref_dot(const RefRaw<T>& r, const float* x) {
                 const uint32_t q = (i < 16u ? (v & 15u) : (v >> 4)) | (((qh >> i) & 1u) << 4);
                 const float w = T == T_Q5_0 ? __fmul_rn(static_cast<float>(static_cast<int>(q) - 16), d)
                                             : __fadd_rn(__fmul_rn(static_cast<float>(q), d), m);
-                s = __fadd_rn(s, __fmul_rn(w, xs[j]));
+#pragma unroll
+                for (int n = 0; n < N; ++n) s[n] = __fadd_rn(s[n], __fmul_rn(w, at4(xv[n], j)));
             }
         }
     } else if constexpr (T == T_Q2_K || T == T_Q3_K) {
@@ -455,11 +489,15 @@ __device__ float ref_dot(const RefRaw<T>& r, const float* x) {
             }
             d = r.d;
         }
-        X8 xa = ldx8(x4, 0u), xb;
+        X8 xa[N], xb[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n) xa[n] = ldx8(x4[n], 0u);
 #pragma unroll
         for (uint32_t g = 0; g < 16; ++g) {  // 16-element groups in element order
-            if ((g & 1u) == 0u && g < 14u)  // the next two groups' x ahead of this pair
-                xb = ldx8(x4 + zero_after(s), 4u * (g + 2u));
+            if ((g & 1u) == 0u && g < 14u) {  // the next two groups' x ahead of this pair
+#pragma unroll
+                for (int n = 0; n < N; ++n) xb[n] = ldx8(x4[n] + zero_after(s[n]), 4u * (g + 2u));
+            }
             const uint32_t h = g / 8u, sh = (g % 8u) / 2u, t = g % 2u;
             const uint32_t scb = (sw[g / 4u] >> (8u * (g % 4u))) & 0xffu;
             float mul, off;
@@ -473,8 +511,6 @@ __device__ float ref_dot(const RefRaw<T>& r, const float* x) {
 #pragma unroll
             for (uint32_t k = 0; k < 4; ++k) {
                 const uint32_t qv = qw[(32u * h + 16u * t) / 4u + k];
-                const float4 xv = xa.v[4u * (g & 1u) + k];
-                const float xs[4] = {xv.x, xv.y, xv.z, xv.w};
 #pragma unroll
                 for (uint32_t j = 0; j < 4; ++j) {
                     const uint32_t q = (qv >> (8u * j + 2u * sh)) & 3u;
@@ -485,27 +521,42 @@ __device__ float ref_dot(const RefRaw<T>& r, const float* x) {
                         const uint32_t hb = (r.hw[(16u * t) / 4u + k] >> (8u * j + 4u * h + sh)) & 1u;
                         w = __fmul_rn(mul, static_cast<float>(static_cast<int>(q) - (hb ? 0 : 4)));
                     }
-                    s = __fadd_rn(s, __fmul_rn(w, xs[j]));
+#pragma unroll
+                    for (int n = 0; n < N; ++n)
+                        s[n] = __fadd_rn(s[n], __fmul_rn(w, at4(xa[n].v[4u * (g & 1u) + k], j)));
                 }
             }
-            if ((g & 1u) == 1u && g < 15u) xa = xb;
+            if ((g & 1u) == 1u && g < 15u) {
+#pragma unroll
+                for (int n = 0; n < N; ++n) xa[n] = xb[n];
+            }
         }
     } else {  // Q4_0: low nibbles are elements 0..15, high 16..31
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
-            const float4 xv = x4[k];
-            const float xs[4] = {xv.x, xv.y, xv.z, xv.w};
+            float4 xv[N];
+#pragma unroll
+            for (int n = 0; n < N; ++n) xv[n] = x4[n][k];
 #pragma unroll
             for (uint32_t m = 0; m < 4; ++m) {
                 const uint32_t i = 4u * k + m, byte = i & 15u;
                 const uint32_t v = (r.w[byte / 4u] >> (8u * (byte % 4u))) & 0xffu;
                 const int q = static_cast<int>(i < 16u ? (v & 15u) : (v >> 4)) - 8;
-                s = __fadd_rn(s, __fmul_rn(xs[m], static_cast<float>(q)));
+#pragma unroll
+                for (int n = 0; n < N; ++n)
+                    s[n] = __fadd_rn(s[n], __fmul_rn(at4(xv[n], m), static_cast<float>(q)));
             }
         }
-        s = __fmul_rn(r.d, s);
+#pragma unroll
+        for (int n = 0; n < N; ++n) s[n] = __fmul_rn(r.d, s[n]);
     }
-    return s;
+}
+
+template <int T>
+__device__ float ref_dot(const RefRaw<T>& r, const float* x) {
+    float s[1];
+    ref_dots<T, 1>(r, x, 0u, s);
+    return s[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -666,6 +717,33 @@ __device__ uint32_t ref_route_block(const RefRouteIn& R, uint32_t route, bool le
     return sh.sel[route];
 }
 
+// The matrix that a workgroup (or, paired, half of one) takes rows of, and its place
+// among that matrix's workgroups.
+struct RefRows {
+    const uint8_t* W;
+    uint64_t slice_bytes;
+    uint32_t rows, bx;
+    float* y;
+};
+
+__device__ __forceinline__ RefRows ref_rows(const RefMatvecArgs& a, bool paired, uint32_t mat) {
+    RefRows R{a.W, a.slice_bytes, a.rows, blockIdx.x, a.y};
+    if (paired) {
+        R.W = a.seg[mat].W;
+        R.slice_bytes = a.seg[mat].slice_bytes;
+        R.rows = a.seg[mat].rows;
+    } else if (a.nseg) {
+#pragma unroll
+        for (uint32_t j = 0; j < kMaxRefSegs; ++j) {
+            if (j < a.nseg && blockIdx.x >= a.seg[j].block0) {
+                R = RefRows{a.seg[j].W, a.seg[j].slice_bytes, a.seg[j].rows,
+                            blockIdx.x - a.seg[j].block0, a.seg[j].y};
+            }
+        }
+    }
+    return R;
+}
+
 // ---------------------------------------------------------------------------
 // y[route][row] for rows of W (route: the expert slice ids[route], or the one
 // routing selects), x[route] staged in LDS -- or, with x_up, the SwiGLU
@@ -678,20 +756,8 @@ __device__ uint32_t ref_route_block(const RefRouteIn& R, uint32_t route, bool le
 // half the same rows of up, and the row sums become the SwiGLU activations
 // g / (1 + expf(-g)) * u (src/qwen3_moe_runner.cpp:682-684), bit for bit
 // what staging them in the down projection computes.
-template <int T, bool BATCH>
+template <int T>
 __global__ __launch_bounds__(256) void k_ref_matvec(RefMatvecArgs a) {
-    if constexpr (BATCH) {  // position blockIdx.z of a prompt chunk
-        const uint64_t off = blockIdx.z * a.tok;
-        a.x += off;
-        if (a.y) a.y += off;
-        if (a.ids) a.ids += off;
-        if (a.act) a.act += off;
-#pragma unroll
-        for (uint32_t j = 0; j < kMaxRefSegs; ++j) a.seg[j].y += off;
-        a.norm.w = nullptr;
-        a.route.logits = nullptr;
-        a.x_up = nullptr;
-    }
     // xs [in], part [256]; with a norm also sq [chain_floats(in)], wb [in]
     extern __shared__ __attribute__((aligned(64))) float lds[];
     __shared__ RouteShared rsh;
@@ -702,28 +768,11 @@ __global__ __launch_bounds__(256) void k_ref_matvec(RefMatvecArgs a) {
     const bool paired = a.act != nullptr;
     const uint32_t mat = paired ? tid / 128u : 0u, lt = paired ? tid % 128u : tid;
     const uint32_t nb = a.in / BE, rpw = (paired ? 128u : 256u) / nb;
-    const uint8_t* W = a.W;
-    uint64_t row_bytes = a.row_bytes, slice_bytes = a.slice_bytes;
-    uint32_t rows = a.rows, bx = blockIdx.x;
-    float* y = a.y;
-    if (paired) {
-        W = a.seg[mat].W;
-        row_bytes = a.seg[mat].row_bytes;
-        slice_bytes = a.seg[mat].slice_bytes;
-        rows = a.seg[mat].rows;
-    } else if (a.nseg) {
-#pragma unroll
-        for (uint32_t j = 0; j < kMaxRefSegs; ++j) {
-            if (j < a.nseg && blockIdx.x >= a.seg[j].block0) {
-                W = a.seg[j].W;
-                row_bytes = a.seg[j].row_bytes;
-                slice_bytes = a.seg[j].slice_bytes;
-                rows = a.seg[j].rows;
-                y = a.seg[j].y;
-                bx = blockIdx.x - a.seg[j].block0;
-            }
-        }
-    }
+    const RefRows R = ref_rows(a, paired, mat);
+    const uint8_t* W = R.W;
+    const uint64_t slice_bytes = R.slice_bytes;
+    const uint32_t rows = R.rows, bx = R.bx;
+    float* y = R.y;
     float* xs = lds;  // padded: block b at b * (BE + 4)
     float* part = lds + xpad_floats<BE>(a.in);
     const uint32_t row0 = bx * rpw, lr = lt / nb, b = lt % nb, row = row0 + lr;
@@ -797,6 +846,143 @@ __global__ __launch_bounds__(256) void k_ref_matvec(RefMatvecArgs a) {
         y[static_cast<uint64_t>(r) * a.y_stride + row0 + tid] = acc;
     }
 }
+
+// The same rows for the positions of a prompt chunk.  A workgroup loads its blocks
+// once and takes the inputs that use them two at a time: all positions of its share
+// (blockIdx.z) of a plain matrix; with ids the routes to expert blockIdx.y, or,
+// where the chunk is too short to share experts, route blockIdx.y alone.
+// Bound by the element chains, about 7 instructions a weight of which two are the
+// input's own: pairs halve the others and give each lane two chains to interleave,
+// and the loop spares the reload and the wait for it.  64 positions, hidden 2048,
+// 128 experts, against one workgroup per position and route: Q4_K 305 -> 123 us a
+// launch (q/k/v, o, gate/up), Q6_K down 366 -> 168.
+constexpr uint32_t kRefChunkWgs = 1024;
+// Inputs at a time (Q2_K's and Q3_K's unpacking leaves no registers for a second).
+constexpr uint32_t ref_chunk_inputs(int type) { return type == T_Q2_K || type == T_Q3_K ? 1u : 2u; }
+constexpr uint32_t kRefChunkRoutes = kRefPromptTokens * kMaxRefTopK;
+template <int T>
+__global__ __launch_bounds__(256) void k_ref_matvec_chunk(RefMatvecArgs a, uint32_t routes) {
+    extern __shared__ __attribute__((aligned(64))) float lds[];  // xs [NX][padded in]
+    constexpr uint32_t NX = ref_chunk_inputs(T);
+    __shared__ float part[2][256], gu[2][256];
+    __shared__ uint16_t list[kRefChunkRoutes];  // per wave a quarter
+    __shared__ uint32_t found[4];
+    constexpr uint32_t BE = RefBlock<T>::BE;
+    const uint32_t tid = threadIdx.x;
+    const bool paired = a.act != nullptr;
+    const uint32_t mat = paired ? tid / 128u : 0u, lt = paired ? tid % 128u : tid;
+    const uint32_t nb = a.in / BE, rpw = (paired ? 128u : 256u) / nb;
+    const RefRows R = ref_rows(a, paired, mat);
+    const uint32_t row0 = R.bx * rpw, lr = lt / nb, b = lt % nb, row = row0 + lr;
+    const bool active = lr < rpw && row < R.rows;
+    const uint64_t nblk = static_cast<uint64_t>(R.rows) * nb;
+    const bool grouped = a.n_slices != 0u, direct = a.ids && !grouped;
+    const uint32_t n = a.tokens * routes;
+    uint64_t slice = 0;
+    if (grouped) slice = blockIdx.y;
+    if (direct) slice = a.ids[blockIdx.y / routes * a.tok + blockIdx.y % routes];
+    RefRaw<T> raw;
+    ref_load<T>(QRow{R.W + slice * R.slice_bytes, nblk, static_cast<uint64_t>(active ? row : 0u) * nb}, b, raw);
+    uint32_t count = n, quarter = 0;
+    if (grouped) {
+        const uint32_t w = tid / 64u, lane = tid % 64u;
+        quarter = (n + 255u) / 256u * 64u;
+        uint32_t at = w * quarter;
+        for (uint32_t j0 = w * quarter; j0 < min((w + 1u) * quarter, n); j0 += 64u) {
+            const uint32_t j = j0 + lane;
+            const bool hit = j < n && a.ids[j / routes * a.tok + j % routes] == slice;
+            const uint64_t m = __ballot(hit);
+            if (hit) list[at + __popcll(m & ((1ull << lane) - 1ull))] = static_cast<uint16_t>(j);
+            at += __popcll(m);
+        }
+        if (lane == 0u) found[w] = at - w * quarter;
+        __syncthreads();
+        count = found[0] + found[1] + found[2] + found[3];
+    }
+    // the k-th input of this matrix, as position * routes + route
+    auto input = [&](uint32_t k) -> uint32_t {
+        if (direct) return blockIdx.y;
+        if (!grouped) return k;
+        uint32_t w = 0;
+        while (k >= found[w]) k -= found[w++];
+        return list[w * quarter + k];
+    };
+    const uint32_t share = (count + gridDim.z - 1u) / gridDim.z, lo = blockIdx.z * share;
+    const uint32_t hi = direct ? 1u : min(lo + share, count);
+    const uint32_t xw = xpad_floats<BE>(a.in), n4 = a.in / 4u;
+    for (uint32_t k = lo; k < hi; k += NX) {
+        const bool two = NX == 2u && k + 1u < hi;  // uniform
+        uint64_t xo[2], yo[2];
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j) {
+            const uint32_t e = input(j && two ? k + 1u : k), t = e / routes, r = e % routes;
+            xo[j] = t * a.tok + static_cast<uint64_t>(r) * a.x_stride;
+            yo[j] = t * a.tok + static_cast<uint64_t>(r) * a.y_stride;
+        }
+        const f32x4* x0 = reinterpret_cast<const f32x4*>(a.x + xo[0]);
+        const f32x4* x1 = reinterpret_cast<const f32x4*>(a.x + xo[1]);
+        for (uint32_t base = 0; base < n4; base += 512u) {
+            const uint32_t i0 = base + tid, i1 = i0 + 256u;
+            const f32x4 v0 = x0[i0 < n4 ? i0 : 0u], v1 = x0[i1 < n4 ? i1 : 0u];
+            f32x4 u0 = v0, u1 = v1;
+            if (two) {
+                u0 = x1[i0 < n4 ? i0 : 0u];
+                u1 = x1[i1 < n4 ? i1 : 0u];
+            }
+            if (i0 < n4) *reinterpret_cast<f32x4*>(lds + xpad<BE>(4u * i0)) = v0;
+            if (i1 < n4) *reinterpret_cast<f32x4*>(lds + xpad<BE>(4u * i1)) = v1;
+            if (two && i0 < n4) *reinterpret_cast<f32x4*>(lds + xw + xpad<BE>(4u * i0)) = u0;
+            if (two && i1 < n4) *reinterpret_cast<f32x4*>(lds + xw + xpad<BE>(4u * i1)) = u1;
+        }
+        __syncthreads();
+        if constexpr (T == T_Q2_K || T == T_Q3_K) {
+            // unpack in each round: kept unpacked over the loop, the weights take every
+            // register there is
+#pragma unroll
+            for (uint32_t i = 0; i < 16; ++i) asm volatile("" : "+v"(raw.qw[i]));
+            if constexpr (T == T_Q3_K) {
+#pragma unroll
+                for (uint32_t i = 0; i < 8; ++i) asm volatile("" : "+v"(raw.hw[i]));
+            }
+        }
+        if (active) {
+            const float* xb = lds + b * (BE + 4u);
+            if (NX == 2u && two) {
+                float s[2];
+                ref_dots<T, 2>(raw, xb, xw, s);
+                part[0][tid] = s[0];
+                part[1][tid] = s[1];
+            } else {
+                float s[1];
+                ref_dots<T, 1>(raw, xb, 0u, s);
+                part[0][tid] = s[0];
+            }
+        }
+        __syncthreads();
+        // the row sums, one per lane: (input, [gate or up,] row)
+        const uint32_t per = paired ? 2u * rpw : rpw;
+        for (uint32_t i = tid; i < (two ? 2u * per : per); i += 256u) {
+            const uint32_t j = i / per, q = i % per, first = paired ? 128u * (q / rpw) + q % rpw * nb : q * nb;
+            float acc = 0.0f;
+            for (uint32_t c = 0; c < nb; ++c) acc = __fadd_rn(acc, part[j][first + c]);
+            if (paired)
+                gu[j][q] = acc;
+            else if (row0 + q < R.rows)
+                R.y[yo[j] + row0 + q] = acc;
+        }
+        if (paired) {
+            __syncthreads();
+            for (uint32_t i = tid; i < (two ? 2u * rpw : rpw); i += 256u) {
+                const uint32_t j = i / rpw, q = i % rpw;
+                if (row0 + q >= R.rows) continue;
+                const float g = gu[j][q], u = gu[j][rpw + q];
+                a.act[yo[j] + row0 + q] = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf_libm(-g, a.expf))), u);
+            }
+        }
+        // the next round's first barrier keeps its part and gu behind these reads
+    }
+}
+
 
 // F32 linear: 0 + dot_f32(w_row, x), one 256-thread workgroup per row: x (or
 // RMSNorm of the residual stream) staged in LDS, the products formed in
@@ -1340,16 +1526,34 @@ uint32_t ref_block_elems(uint32_t type) {
                : 256u;
 }
 
+// Experts are shared by positions from one route per expert on average.  The inputs of
+// a matrix are split over workgroups where its rows alone do not fill the chip twice
+// over.
+template <int T>
+hipError_t ref_chunk_t(RefMatvecArgs a, uint32_t blocks, uint32_t routes, hipStream_t s) {
+    if (a.norm.w || a.route.logits || a.x_up || a.tokens > kRefPromptTokens || routes > kMaxRefTopK ||
+        (a.ids ? a.n_slices == 0u : routes != 1u))
+        return hipErrorInvalidValue;
+    const size_t lds = ref_chunk_inputs(T) * xpad_floats<RefBlock<T>::BE>(a.in) * sizeof(float);
+    uint32_t matrices = 1, split = 0;
+    if (a.ids && a.tokens * routes < a.n_slices) {
+        matrices = a.tokens * routes;
+        a.n_slices = 0;
+        split = 1;
+    } else if (a.ids) {
+        matrices = a.n_slices;
+    }
+    if (!split) split = std::min((kRefChunkWgs + blocks * matrices - 1u) / (blocks * matrices), a.tokens);
+    hipLaunchKernelGGL(k_ref_matvec_chunk<T>, dim3(blocks, matrices, split), dim3(256), lds, s, a, routes);
+    return hipGetLastError();
+}
+
 template <int T>
 hipError_t ref_matvec_t(const RefMatvecArgs& a, uint32_t blocks, uint32_t routes, hipStream_t s) {
+    if (a.tokens) return ref_chunk_t<T>(a, blocks, routes, s);
     size_t lds = (xpad_floats<RefBlock<T>::BE>(a.in) + 256u) * sizeof(float);
     if (a.norm.w) lds += (chain_floats(a.in) + a.in) * sizeof(float);
-    if (a.tokens > 1u) {
-        if (a.norm.w || a.route.logits || a.x_up) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_ref_matvec<T, true>), dim3(blocks, routes, a.tokens), dim3(256), lds, s, a);
-    } else {
-        hipLaunchKernelGGL((k_ref_matvec<T, false>), dim3(blocks, routes), dim3(256), lds, s, a);
-    }
+    hipLaunchKernelGGL(k_ref_matvec<T>, dim3(blocks, routes), dim3(256), lds, s, a);
     return hipGetLastError();
 }
 
@@ -1400,7 +1604,7 @@ hipError_t launch_ref_matvec(uint32_t type, const RefMatvecArgs& a, uint32_t rou
         if (a.route.logits || a.x_up || a.nseg) return hipErrorInvalidValue;
         size_t lds = (chain_floats(a.in) + a.in) * sizeof(float);
         if (a.norm.w) lds += (chain_floats(a.in) + a.in) * sizeof(float);
-        if (a.tokens > 1u) {
+        if (a.tokens) {
             if (a.norm.w) return hipErrorInvalidValue;
             hipLaunchKernelGGL(k_ref_linear_f32<true>, dim3(a.rows, routes, a.tokens), dim3(256), lds, s, a);
         } else {
@@ -1494,7 +1698,7 @@ bool ref_prompt_supported(const ModelArgs& a, const ModelLayer* layers) {
 // launch_ref_step's layers for a chunk of positions: the same arithmetic per
 // position, its serial chains side by side across positions instead of one after
 // the other.  (2 layers of hidden 2048, 128 experts, 32-token prompt and 16 new
-// tokens: 8.53 -> 5.47 ms.)
+// tokens: 8.53 -> 4.76 ms, of which the 16 steps are 3.0.)
 hipError_t launch_ref_prompt_chunk(const ModelArgs& a, const ModelLayer* layers, uint32_t* ids,
                                    float* probs, uint32_t tokens, uint64_t tok, hipStream_t s) {
     const uint32_t qd = a.heads * a.head_dim, kd = a.kv_heads * a.head_dim, H = a.hidden;
@@ -1557,6 +1761,7 @@ hipError_t launch_ref_prompt_chunk(const ModelArgs& a, const ModelLayer* layers,
         gu.x = a.normed;
         gu.y_stride = m.ffn;
         gu.ids = ids;
+        gu.n_slices = m.n_experts;
         gu.act = g;
         gu.expf = a.expf;
         if ((err = launch_ref_gate_up_act(m.gate_type, gu, RefSeg{m.gate, m.gate_row, m.gate_slice, m.ffn, 0, g},
@@ -1564,6 +1769,7 @@ hipError_t launch_ref_prompt_chunk(const ModelArgs& a, const ModelLayer* layers,
             return err;
         RefMatvecArgs d = base;
         d.ids = ids;
+        d.n_slices = m.n_experts;
         d.W = m.down;
         d.row_bytes = m.down_row;
         d.slice_bytes = m.down_slice;

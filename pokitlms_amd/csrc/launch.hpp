@@ -335,10 +335,12 @@ struct RefMatvecArgs {
     LibmExpf expf;
     RefNormIn norm;           // norm.w set: x is RMSNorm(norm.x + norm.res) * norm.w
     RefRouteIn route;         // route.logits set: the expert slices come from routing
-    // the same for `tokens` positions (grid z): x, y, ids and act of position t are
-    // t * tok words on; no norm, routing or x_up then
-    uint32_t tokens = 1;
+    // Set: the same for `tokens` positions of a prompt chunk; x, y, ids and act of
+    // position t are t * tok words on.  ids then choose from n_slices expert slices.
+    // No norm, routing or x_up.
+    uint32_t tokens = 0;
     uint64_t tok = 0;
+    uint32_t n_slices = 0;
 };
 bool ref_matvec_supported(uint32_t type, uint32_t in);
 hipError_t launch_ref_matvec(uint32_t type, const RefMatvecArgs& a, uint32_t routes,

@@ -57,3 +57,41 @@ def test_scratch_leaves_the_bits(hip):
     for i in (0, 1):
         assert np.array_equal(out[i][0], out[i + 2][0])
         assert np.array_equal(out[i][1].view(np.uint32), out[i + 2][1].view(np.uint32))
+
+
+@pytest.mark.parametrize("gtype", (S.Q4_0, S.Q4_1, S.Q5_0, S.Q5_1, S.Q8_0, S.Q2_K, S.Q3_K, S.Q4_K,
+                                   S.Q5_K, S.Q6_K))
+def test_formats(hip, gtype):
+    """Every format of the chunk's matrices (experts: those the MoE block takes): 3 positions take their
+    routes one by one (12 routes, 16 experts), 4 and more share the experts' rows, an
+    odd number of inputs to a matrix ends in a single one."""
+    from pokitlms_amd.model import Qwen3MoeModel
+    m = shape()
+    weights = Qwen3MoeModel.synthetic_weights(hip, m, 31)
+    gen = S.rng(80 + gtype)
+    names = {"attn_q": (512, 512, 0), "attn_k": (512, 256, 0), "attn_v": (512, 256, 0),
+             "attn_output": (512, 512, 0), "ffn_gate_exps": (512, 256, 16),
+             "ffn_up_exps": (512, 256, 16), "ffn_down_exps": (256, 512, 16)}
+    if gtype in (S.Q5_0, S.Q5_1, S.Q2_K, S.Q3_K):
+        names = {k: v for k, v in names.items() if v[2] == 0}
+    for layer in range(m.layers):
+        for name, (inn, out, ne) in names.items():
+            key = f"blk.{layer}.{name}.weight"
+            weights[key].release()
+            rows = S.quant_matrix(gtype, out * max(ne, 1), inn, gen)
+            blocks = rows.reshape(-1, S.BLOCK_BYTES[gtype])
+            flip = gen.integers(0, 2, len(blocks), dtype=np.uint8) << 7
+            for off in S.SCALE_OFFSETS[gtype]:  # half the blocks negated: weights around zero
+                blocks[:, off + 1] ^= flip
+            weights[key] = hip.upload(gtype, inn, out, rows, ne)
+    with Qwen3MoeModel(hip, m, weights) as model:
+        seen = set()
+        for start in (9, 10, 11):
+            first = SM.prompt_tokens(start, 1, m.vocab)
+            steps, _, _ = model.generate(first, 48)
+            seen.update(steps.tolist())
+            seq = np.concatenate((first, steps))
+            for n in (3, 4, 5, 6, 18, 41):
+                got, _, _ = model.generate(seq[:n], 4)
+                assert np.array_equal(got, seq[n:n + 4]), (start, n)
+    assert len(seen) >= 3  # sequences worth comparing
