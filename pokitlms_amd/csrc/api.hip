@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "../../include/pokit_hip.h"
+#include "chunk_scratch.hpp"
 #include "launch.hpp"
 #include "layout.hpp"
 
@@ -1371,14 +1372,7 @@ struct pk_hip_qwen3moe {
     DeviceBuffer<double> row_sum, row_bound;
     DeviceBuffer<uint16_t> kv;
     DeviceBuffer<uint8_t> qkv;  // fast mode: each layer's q, k and v rows back to back
-    // fast mode: scratch of the batched prompt, for chunks of prompt_tokens positions
-    uint8_t* prompt_mem = nullptr;
-    uint32_t prompt_tokens = 0;
-    pk::PromptArgs prompt{};
-    // reference order: per position of a chunk, the step's buffers
-    uint64_t ref_tok = 0;
-    uint32_t* ref_ids = nullptr;
-    float* ref_probs = nullptr;
+    pk::ChunkScratch prompt;    // the batched prompt's scratch; each call lays it out anew
     hipGraphExec_t step_logits = nullptr, step_plain = nullptr;
     hipEvent_t ev[2] = {};
 };
@@ -1421,6 +1415,16 @@ hipGraphExec_t capture_step(pk_hip_qwen3moe* m, bool logits) {
     return exec;
 }
 
+// The prompt's scratch is kept with the model and given back with it.  Where memory
+// for it is short, the prompt takes token steps, which need none.
+uint8_t* prompt_alloc(uint64_t bytes) {
+    uint8_t* mem = nullptr;
+    if (hipMalloc(&mem, bytes) == hipSuccess) return mem;
+    (void)hipGetLastError();
+    return nullptr;
+}
+void prompt_free(uint8_t* mem) { (void)hipFree(mem); }
+
 void release_model(pk_hip_qwen3moe* m) {
     if (m->step_logits) (void)hipGraphExecDestroy(m->step_logits);
     if (m->step_plain) (void)hipGraphExecDestroy(m->step_plain);
@@ -1441,8 +1445,8 @@ void release_model(pk_hip_qwen3moe* m) {
     m->row_bound.release();
     m->kv.release();
     m->qkv.release();
-    if (m->prompt_mem) (void)hipFree(m->prompt_mem);
-    m->prompt_mem = nullptr;
+    if (m->prompt.mem) prompt_free(m->prompt.mem);
+    m->prompt = pk::ChunkScratch{};
 }
 
 // Fewer prompt positions than this go through token steps: a short chunk costs about
@@ -1456,32 +1460,30 @@ constexpr uint32_t kPromptMin = 5;
 // 10318, 3927 against 28236).
 constexpr uint32_t kRefPromptMin = 2;
 
-// The prompt's scratch is kept with the model and given back with it.  False where
-// memory for it is short (the token steps need none).
-bool grow_prompt_mem(pk_hip_qwen3moe* m, uint64_t bytes, uint32_t tokens) {
-    uint8_t* mem = nullptr;
-    if (hipMalloc(&mem, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    if (m->prompt_mem) (void)hipFree(m->prompt_mem);
-    m->prompt_mem = mem;
-    m->prompt_tokens = tokens;
+// Fast mode: scratch for chunks of min(n, kPromptTokens) positions, laid out in a.
+bool prompt_scratch_ready(pk_hip_qwen3moe* m, uint32_t n, pk::PromptArgs& a) {
+    constexpr uint32_t rungs[] = {64, 192, pk::kPromptTokens};
+    auto bytes = [&](uint32_t t) {
+        pk::PromptArgs size{};
+        return pk::prompt_scratch(m->args, m->layers.data(), t, nullptr, size);
+    };
+    if (!pk::chunk_scratch_ready(m->prompt, rungs, 3, n, bytes, prompt_alloc, prompt_free)) return false;
+    pk::prompt_scratch(m->args, m->layers.data(), m->prompt.tokens, m->prompt.mem, a);
     return true;
 }
 
-// Fast mode: scratch for chunks of min(n, kPromptTokens) positions.
-bool prompt_scratch_ready(pk_hip_qwen3moe* m, uint32_t n) {
-    const uint32_t t = std::min(n <= 64 ? 64u : n <= 192 ? 192u : pk::kPromptTokens, pk::kPromptTokens);
-    if (m->prompt_tokens >= t) return true;
-    const uint64_t bytes = pk::prompt_scratch(m->args, m->layers.data(), t, nullptr, m->prompt);
-    if (!grow_prompt_mem(m, bytes, t)) return false;
-    pk::prompt_scratch(m->args, m->layers.data(), t, m->prompt_mem, m->prompt);
-    return true;
-}
+// Reference order: per position of a chunk, the step's buffers.
+struct RefChunk {
+    pk::ModelArgs m;
+    uint32_t* ids;
+    float* probs;
+    uint64_t tok;  // words from one position's buffers to the next's
+};
 
 // Reference order: each position's copy of the step's buffers, 256-byte aligned.
-bool ref_prompt_ready(pk_hip_qwen3moe* m, uint32_t n, pk::ModelArgs& a) {
+bool ref_prompt_ready(pk_hip_qwen3moe* m, uint32_t n, RefChunk& c) {
+    pk::ModelArgs& a = c.m;
+    a = m->args;
     const uint64_t H = a.hidden, qd = uint64_t(a.heads) * a.head_dim, kd = uint64_t(a.kv_heads) * a.head_dim;
     uint64_t ffn = 1;
     for (const pk::ModelLayer& L : m->layers) ffn = std::max<uint64_t>(ffn, L.moe.ffn);
@@ -1495,12 +1497,13 @@ bool ref_prompt_ready(pk_hip_qwen3moe* m, uint32_t n, pk::ModelArgs& a) {
                    k = take(kd), v = take(kd), att = take(qd),
                    scratch = take(pk::ref_scratch_floats(m->cfg.top_k, static_cast<uint32_t>(ffn), a.hidden)),
                    ids = take(16), probs = take(16);
-    const uint32_t t = std::min(n <= 32 ? 32u : pk::kRefPromptTokens, pk::kRefPromptTokens);
-    if (m->prompt_tokens < t && !grow_prompt_mem(m, at * t * sizeof(float), t)) return false;
-    float* p = reinterpret_cast<float*>(m->prompt_mem);
-    m->ref_tok = at;
-    m->ref_ids = reinterpret_cast<uint32_t*>(p + ids);
-    m->ref_probs = p + probs;
+    constexpr uint32_t rungs[] = {32, pk::kRefPromptTokens};
+    auto bytes = [&](uint32_t t) { return at * t * sizeof(float); };
+    if (!pk::chunk_scratch_ready(m->prompt, rungs, 2, n, bytes, prompt_alloc, prompt_free)) return false;
+    float* p = reinterpret_cast<float*>(m->prompt.mem);
+    c.tok = at;
+    c.ids = reinterpret_cast<uint32_t*>(p + ids);
+    c.probs = p + probs;
     a.hidden_state = p + hidden;
     a.hidden_alt = p + alt;
     a.normed = p + normed;
@@ -1769,20 +1772,21 @@ pk_hip_status pk_hip_qwen3moe_generate(pk_hip_qwen3moe* m, const uint32_t* promp
         uint32_t done = 0;
         // all but the last prompt token that the KV window holds, in chunks
         const uint32_t batch = std::min(n_prompt - 1, m->cfg.kv_capacity);
-        pk::ModelArgs chunk = m->args;
+        RefChunk ref;
+        pk::PromptArgs fast{};
         if (batch >= kRefPromptMin && pk::ref_prompt_supported(m->args, m->layers.data()) &&
-            ref_prompt_ready(m, batch, chunk)) {
-            for (; done < batch; done += std::min(batch - done, m->prompt_tokens))
-                check(pk::launch_ref_prompt_chunk(chunk, m->layers.data(), m->ref_ids, m->ref_probs,
-                                                  std::min(batch - done, m->prompt_tokens), m->ref_tok, s),
+            ref_prompt_ready(m, batch, ref)) {
+            for (uint32_t n; done < batch; done += n) {
+                n = std::min(batch - done, m->prompt.tokens);
+                check(pk::launch_ref_prompt_chunk(ref.m, m->layers.data(), ref.ids, ref.probs, n, ref.tok, s),
                       "prompt chunk");
+            }
         } else if (batch >= kPromptMin && pk::prompt_supported(m->args, m->layers.data()) &&
-                   prompt_scratch_ready(m, batch)) {
-            m->prompt.m = m->args;
-            for (; done < batch; done += std::min(batch - done, m->prompt_tokens))
-                check(pk::launch_prompt_chunk(m->prompt, m->layers.data(),
-                                              std::min(batch - done, m->prompt_tokens), done, s),
-                      "prompt chunk");
+                   prompt_scratch_ready(m, batch, fast)) {
+            for (uint32_t n; done < batch; done += n) {
+                n = std::min(batch - done, m->prompt.tokens);
+                check(pk::launch_prompt_chunk(fast, m->layers.data(), n, done, s), "prompt chunk");
+            }
         }
         for (uint32_t i = done; i + 1 < n_prompt; ++i) check(hipGraphLaunch(m->step_plain, s), "prefill step");
         check(hipGraphLaunch(m->step_logits, s), "prefill logits step");
