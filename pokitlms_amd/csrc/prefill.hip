@@ -46,7 +46,8 @@ namespace {
 // product: 275 us for 4096 tokens x 128 rows of 2048, 42 us for 512; so: 116
 // and 21 us, bound by those three instructions; the ranking's second look at what
 // the coarser bound leaves open adds 6 us).  The waves' operands pass
-// through LDS parts of their own; the only barrier is before the waves' sums meet.
+// through LDS parts of their own, ordered within the wave (wave_lds_order); the only
+// barrier is before the waves' sums meet.
 //
 // The bound.  With T_i the exact prefix sums of the products p_i, the serial sum
 // is within u (1 + 2^-10) sum_i |T_i| of S.  In a run of 16 products from prefix O
@@ -135,6 +136,7 @@ __global__ __launch_bounds__(64 * kRtWaves, 4) void k_router_batch(MoePrefillArg
             }
         }
         load(set, k + NS * kRtK);
+        wave_lds_order();  // the lanes read each other's stores
 #pragma unroll
         for (uint32_t c = 0; c < kRtK / 4u; ++c) {
             rf32x4 x[TT], w[TE];
@@ -156,6 +158,7 @@ __global__ __launch_bounds__(64 * kRtWaves, 4) void k_router_batch(MoePrefillArg
                     for (uint32_t e = 0; e < TE; ++e) q[t][e] += fabs(l[t][e]);
             }
         }
+        wave_lds_order();  // and the next stage's stores overwrite what they read
     };
     uint32_t k = 0;
     for (; k + NS * kRtK <= range; k += NS * kRtK)

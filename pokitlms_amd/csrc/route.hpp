@@ -253,6 +253,15 @@ __device__ __forceinline__ WaveRoutes<NS> wave_route(const MoeDecodeArgs& a, con
     return w;
 }
 
+// Between a wave's LDS accesses where its lanes read what others of them wrote, or
+// write over what others read: LDS keeps one wave's accesses in order, the fences
+// keep the compiler from reordering them.  No instruction, no workgroup barrier.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The same ranking and certification by a workgroup of four waves, as
 // counts instead of top_k dependent wave maxima: the rank of expert e is the
 // number of experts whose key exceeds its key.  Wave w ranks experts
@@ -308,11 +317,7 @@ __device__ __forceinline__ void wg_rank(const MoeDecodeArgs& a, const RouteData<
         const uint32_t e = lane + 64u * m;
         kw[e] = e < E ? route_key(static_cast<float>(d.S[m]), e) : 0u;
     }
-    // the wave reads what its other lanes wrote: LDS keeps one wave's
-    // accesses in order, the fences keep the compiler from reordering them
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_order();
     const uint32_t* kh = kw + HK * (lane >> 5);
 #pragma unroll
     for (int p = 0; p < rank_passes<NS>(); ++p) {
