@@ -419,12 +419,12 @@ __device__ __forceinline__ float half_wave_max(float v) {
     return __uint_as_float(max(s[0], s[1]));
 }
 
-// MT x 32 assignments of a tile, from its row row0.  DUAL: gate and up rows n0 .. n0 + 127 over x,
+// MT x 32 assignments of a tile.  DUAL: gate and up rows n0 .. n0 + 127 over x,
 // SwiGLU, activations split for the down GEMM; otherwise down rows n0 .. n0 + 255
 // over the activations, each output row to its (token, route) slot.
 template <int T, bool UNITS, bool DUAL, int MT>
 __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef& tr, uint32_t n0,
-                                          GemmShared& sh, uint32_t row0 = 0u) {
+                                          GemmShared& sh) {
     using W = WTraits<T, UNITS>;
     const MoeDecodeArgs& L = a.layer;
     const uint32_t kdim = DUAL ? L.hidden : L.ffn, ndim = DUAL ? L.ffn : L.hidden;
@@ -469,10 +469,10 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const uint32_t row = pr + 32u * i;
-        asrc[i] = parts + static_cast<uint64_t>(sh.arow[row0 + row]) * kdim * 2u + pc * 8u;
+        asrc[i] = parts + static_cast<uint64_t>(sh.arow[row]) * kdim * 2u + pc * 8u;
         adst[i] = row * kStageRow + ((pc ^ (row & 7u)) * 16u);
-        csrc[i] = DUAL ? nullptr : a.act_scale + static_cast<uint64_t>(sh.arow[row0 + row]) * nst;
-        cinv[i] = DUAL ? 0.0f : 1.0f / sh.scale[row0 + row];
+        csrc[i] = DUAL ? nullptr : a.act_scale + static_cast<uint64_t>(sh.arow[row]) * nst;
+        cinv[i] = DUAL ? 0.0f : 1.0f / sh.scale[row];
     }
     // register sets of stages in flight: with one row block there is room for eight,
     // which small batches need, where little else hides the loads' latency (77
@@ -502,25 +502,28 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
             *reinterpret_cast<u32x4_t*>(sh.st[buf] + adst[i]) = v;
         }
     };
-    // group sums: thread t of the first 4 * 32 MT takes groups 2 (t % 4), + 1 of row t / 4
-    const uint32_t sr = (tid / 4u) < 32u * MT ? tid / 4u : 0u, sg = 2u * (tid % 4u);
-    const float* ssrc = W::kMins ? sums + static_cast<uint64_t>(sh.arow[row0 + sr]) * nst + sg : nullptr;
-    const float sinv = W::kMins ? (W::kMinsF32 ? 1.0f : 0x1p-5f) / sh.scale[row0 + sr] : 0.0f;
+    // group sums: thread t takes groups 2 (t % 4), + 1 of row t / 4; with one row block
+    // the upper half of the threads has none.  For Q4_1 it stores row 0's sums to the
+    // rows that nobody reads all the same: a branch here would split the unrolled
+    // superblock, and the values held across it did not fit the registers (61 spilled
+    // with one row block, 340 with two; none without the branch).  The other formats
+    // fit better with it.
+    const uint32_t dr = tid / 4u, sr = dr < 32u * MT ? dr : 0u, sg = 2u * (tid % 4u);
+    const float* ssrc = W::kMins ? sums + static_cast<uint64_t>(sh.arow[sr]) * nst + sg : nullptr;
+    const float sinv = W::kMins ? (W::kMinsF32 ? 1.0f : 0x1p-5f) / sh.scale[sr] : 0.0f;
     float2 sv = make_float2(0.0f, 0.0f);
     auto load_sums = [&](uint32_t sb) {
         if constexpr (W::kMins) sv = *reinterpret_cast<const float2*>(ssrc + 8u * (sb < nsb ? sb : nsb - 1u));
     };
     auto store_sums = [&](uint32_t buf) {
+        if (T != T_Q4_1 && tid >= 128u * MT) return;
         if constexpr (W::kMinsF32) {
-            if (tid < 128u * MT)
-                *reinterpret_cast<float2*>(sh.xs[buf] + sr * 32u + sg * 4u) = make_float2(sv.x * sinv, sv.y * sinv);
+            *reinterpret_cast<float2*>(sh.xs[buf] + dr * 32u + sg * 4u) = make_float2(sv.x * sinv, sv.y * sinv);
         } else if constexpr (W::kMins) {
             uint32_t hi, lo;
             split_pair(sv.x * sinv, sv.y * sinv, hi, lo);
-            if (tid < 128u * MT) {
-                *reinterpret_cast<uint32_t*>(sh.xs[buf] + sr * 32u + sg * 2u) = hi;
-                *reinterpret_cast<uint32_t*>(sh.xs[buf] + sr * 32u + 16u + sg * 2u) = lo;
-            }
+            *reinterpret_cast<uint32_t*>(sh.xs[buf] + dr * 32u + sg * 2u) = hi;
+            *reinterpret_cast<uint32_t*>(sh.xs[buf] + dr * 32u + 16u + sg * 2u) = lo;
         }
     };
     // A fragments: piece (plane, 2 kq + h or 2 h + kq) of row ln (+ 32)
@@ -677,7 +680,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         for (int m = 0; m < MT; ++m) {
 #pragma unroll
             for (uint32_t r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
+                const uint32_t row = 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
                 const float s = sh.scale[row];
                 const float g = acc[m][0][r] * (u0 * s), u = acc[m][1][r] * (u1 * s);
                 const float v = (g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))) * u;
@@ -705,7 +708,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (uint32_t r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
+                const uint32_t row = 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
                 if (row < tr.rows) {
                     const float s = sh.scale[row];
                     float* o = out + static_cast<uint64_t>(sh.oslot[row]) * ndim + n0 + wave * 32u + ln;
@@ -746,12 +749,7 @@ __global__ __launch_bounds__(256, 2) void k_expert_gemm(MoePrefillArgs a) {
         if (tid % 4u == 0u) sh.scale[row] = m;
     }
     __syncthreads();
-    if constexpr (T == T_Q4_1) {  // its scales and mins leave no registers for two row blocks
-        for (uint32_t row0 = 0; row0 < tr.rows; row0 += 32u) {
-            if (row0) __syncthreads();
-            gemm_tile<T, UNITS, DUAL, 1>(a, tr, yb * nblk, sh, row0);
-        }
-    } else if (tr.rows > 32u) {
+    if (tr.rows > 32u) {
         gemm_tile<T, UNITS, DUAL, 2>(a, tr, yb * nblk, sh);
     } else {
         gemm_tile<T, UNITS, DUAL, 1>(a, tr, yb * nblk, sh);
