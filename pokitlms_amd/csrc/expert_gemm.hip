@@ -18,8 +18,8 @@
 // as whole lines through LDS, fragments read half a step ahead with a barrier
 // every second step, and both: the same gate/up time, slower down.)  Error against
 // float64 on the same inputs, before and after: Q4_K/Q6_K 3.8e-6 -> 7.8e-7,
-// Q6_K 9.7e-7 -> 3.6e-7, Q5_K 4.4e-7 -> 4.0e-7, Q8_0 4.4e-7 -> 3.0e-7, Q4_0
-// 4.4e-7 -> 2.9e-7, Q4_1 4.4e-7 -> 4.0e-7.
+// Q6_K 9.7e-7 -> 3.6e-7, Q5_K 4.4e-7 -> 3.6e-7, Q8_0 4.4e-7 -> 3.0e-7, Q4_0
+// 4.4e-7 -> 2.9e-7, Q4_1 4.6e-7 -> 4.0e-7.
 #include <math.h>
 
 #include "gemm_split.hpp"
@@ -71,14 +71,20 @@ __device__ __forceinline__ uint32_t pk_mul_f16(uint32_t a, f16x2 b) {
 //    rescaled by d_prev / d once per 256 values.  The mins' term is one more
 //    MFMA per superblock: the eight integer mins against the eight group sums of
 //    x (split hi and lo, 16 operand values).
-//  * Q5_K, and Q4_K in the prompt's projections: q - 16 (q - 8) and a partial sum per
-//    superblock, the rest of the mins' term (16 d sc - dmin m) times the FP32 group
-//    sums on FP32 MFMA.  As kUnits, Q5_K had 6.1e-7 against the 3.6e-7 of the kernel
-//    before it (the larger quants leave more to cancel against the mins), and Q4_K
-//    projections at 8.7e-7 (4.0e-7 so) put the whole model's logits 15% further from
-//    float64, as fewer FP16 roundings of k then agree; the MoE block's gate/up keeps
-//    the units, 472 against 557 us at 4096 tokens and five times more exact than the
-//    bf16 parts before.
+//  * Q5_K, and Q4_K in the prompt's projections: q - 16 (q - 8), the rest of the mins'
+//    term (16 d sc - dmin m) times the FP32 group sums on FP32 MFMA.  With two row
+//    blocks each step's sum goes into the accumulator by an FMA with d, as the other
+//    formats' do; with one there are registers for sums over the superblock, the high
+//    and the low halves' apart (kHalves), which is a chain less to wait for.  A single
+//    sum of both over the superblock was 20% further from float64 at hidden 512 (Q5_K
+//    3.5e-7 against 2.9e-7; 1024: 3.7e-7 against 3.2e-7, 2048: 4.5e-7 against 4.3e-7) and
+//    spilled 13 to 23 registers (2048 tokens 735 -> 701 us without, 77 tokens level).
+//    As kUnits, Q5_K had 6.1e-7 (the larger quants leave more to cancel against the
+//    mins), and Q4_K projections at 8.7e-7 put the whole model's logits 15% further from
+//    float64, as fewer FP16 roundings of k then agree; the MoE block's gate/up keeps the
+//    units, 472 against 557 us at 4096 tokens: in the prompt they change nothing of the
+//    logits' error, which is the projections' (over 294 prompts of 1 to 4 layers it is
+//    0.92 of that of one token step per position).
 //
 // The others: quants as exact fp16 integers around zero (1024 + q by or-ing the
 // exponent in, minus 1024 and the offset), and per scale group (32 values;
@@ -276,6 +282,7 @@ __device__ __forceinline__ void wfrag(const WRaw<T>& r, const WHead<T>& hd, uint
                 w[2u * i + 1u] = pk_fma16(w[2u * i + 1u], k4096, mid);
             }
         }
+        if constexpr (!WTraits<T, UNITS>::kUnits) ds[0] = ds[1] = hd.d;
     } else if constexpr (T == T_Q6_K) {
         const uint32_t hh = j / 4u, g = j % 4u;
         uint32_t ql[4], qh[4];
@@ -476,8 +483,9 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     }
     // register sets of stages in flight: with one row block there is room for eight,
     // which small batches need, where little else hides the loads' latency (77
-    // tokens, 64 experts: gate/up 45 -> 42 us; 512 tokens 119 -> 117)
-    constexpr uint32_t NS = MT == 1 ? 8u : 2u;
+    // tokens, 64 experts: gate/up 45 -> 42 us; 512 tokens 119 -> 117); Q5_K's down has
+    // room for four
+    constexpr uint32_t NS = MT == 1 ? (T == T_Q5_K && !DUAL ? 4u : 8u) : 2u;
     u32x4_t av[NS][MT];
     float ac[NS][MT];
     const uint32_t last = 8u * nsb - 1u;
@@ -503,11 +511,11 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         }
     };
     // group sums: thread t takes groups 2 (t % 4), + 1 of row t / 4; with one row block
-    // the upper half of the threads has none.  For Q4_1 it stores row 0's sums to the
-    // rows that nobody reads all the same: a branch here would split the unrolled
-    // superblock, and the values held across it did not fit the registers (61 spilled
-    // with one row block, 340 with two; none without the branch).  The other formats
-    // fit better with it.
+    // the upper half of the threads has none.  It stores row 0's sums to the rows that
+    // nobody reads all the same: a branch here would split the unrolled superblock, and
+    // the values held across it do not fit the registers (Q4_1: 61 spilled with one row
+    // block, 340 with two; none without the branch).  kUnits, with no FMA per step,
+    // fits better with it (208 registers against 256 and 25 spilled).
     const uint32_t dr = tid / 4u, sr = dr < 32u * MT ? dr : 0u, sg = 2u * (tid % 4u);
     const float* ssrc = W::kMins ? sums + static_cast<uint64_t>(sh.arow[sr]) * nst + sg : nullptr;
     const float sinv = W::kMins ? (W::kMinsF32 ? 1.0f : 0x1p-5f) / sh.scale[sr] : 0.0f;
@@ -516,7 +524,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         if constexpr (W::kMins) sv = *reinterpret_cast<const float2*>(ssrc + 8u * (sb < nsb ? sb : nsb - 1u));
     };
     auto store_sums = [&](uint32_t buf) {
-        if (T != T_Q4_1 && tid >= 128u * MT) return;
+        if (W::kUnits && tid >= 128u * MT) return;
         if constexpr (W::kMinsF32) {
             *reinterpret_cast<float2*>(sh.xs[buf] + dr * 32u + sg * 4u) = make_float2(sv.x * sinv, sv.y * sinv);
         } else if constexpr (W::kMins) {
@@ -547,7 +555,8 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     load_act(0u, 8u * sb0 + NS);
     __syncthreads();
 
-    f32x16 acc[MT][2], part[MT][2];  // part: Q5_K, the superblock's sums
+    f32x16 acc[MT][2], half[2][2];  // half: kHalves, the superblock's sums of the high and low parts
+    constexpr bool kHalves = MT == 1 && W::kSuper && !W::kUnits;
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = f32x16{};
     float dcur[2] = {1.0f, 1.0f};
@@ -591,48 +600,53 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
                     hd[i].cn[j / 2u] = j & 1u ? (kq ? m : hd[i].cn[j / 2u]) : m;
                 }
             }
-            if constexpr (W::kSuper) {
-                auto& c = W::kUnits ? acc : part;
-                if (!W::kUnits && j == 0u) {
-#pragma unroll
-                    for (int m = 0; m < MT; ++m) c[m][0] = c[m][1] = f32x16{};
-                }
+            if constexpr (W::kUnits) {
 #pragma unroll
                 for (uint32_t h = 0; h < 2; ++h)
 #pragma unroll
                     for (int m = 0; m < MT; ++m) {
                         const f16x8 lo = afrag(buf, m, 1u, h), hi = afrag(buf, m, 0u, h);
-                        c[m][0] = mfma(lo, b[0][h], c[m][0]);
-                        c[m][1] = mfma(lo, b[1][h], c[m][1]);
-                        c[m][0] = mfma(hi, b[0][h], c[m][0]);
-                        c[m][1] = mfma(hi, b[1][h], c[m][1]);
+                        acc[m][0] = mfma(lo, b[0][h], acc[m][0]);
+                        acc[m][1] = mfma(lo, b[1][h], acc[m][1]);
+                        acc[m][0] = mfma(hi, b[0][h], acc[m][0]);
+                        acc[m][1] = mfma(hi, b[1][h], acc[m][1]);
                     }
-                if constexpr (!W::kUnits) if (j == 7u) {
+            } else if constexpr (kHalves) {
 #pragma unroll
-                    for (int m = 0; m < MT; ++m)
+                for (uint32_t k = 0; k < 4; ++k) {  // hi and lo of the first fragment, then of the second
+                    const uint32_t h = k / 2u, p = k & 1u;
+                    const f16x8 f = afrag(buf, 0u, p, h);
 #pragma unroll
-                        for (uint32_t i = 0; i < 2; ++i)
+                    for (uint32_t i = 0; i < 2; ++i)
+                        half[i][p] = mfma(f, b[i][h], j == 0u && h == 0u ? f32x16{} : half[i][p]);
+                }
+                if (j == 7u) {
 #pragma unroll
-                            for (uint32_t r = 0; r < 16; ++r)
-                                acc[m][i][r] = __builtin_fmaf(hd[i].d, c[m][i][r], acc[m][i][r]);
+                    for (uint32_t i = 0; i < 2; ++i)
+#pragma unroll
+                        for (uint32_t r = 0; r < 16; ++r)
+                            acc[0][i][r] = __builtin_fmaf(hd[i].d, half[i][0][r] + half[i][1][r], acc[0][i][r]);
                 }
             } else {
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
-                    f32x16 P, Q;
+                    f32x16 P[2];
 #pragma unroll
-                    for (uint32_t h = 0; h < 2; ++h) {
-                        const f16x8 lo = afrag(buf, m, 1u, h), hi = afrag(buf, m, 0u, h);
-                        const bool first = W::kGroup == 16u || h == 0u;
-                        P = mfma(lo, b[0][h], first ? f32x16{} : P);
-                        Q = mfma(lo, b[1][h], first ? f32x16{} : Q);
-                        P = mfma(hi, b[0][h], P);
-                        Q = mfma(hi, b[1][h], Q);
-                        if (W::kGroup == 16u || h == 1u) {
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        // group 32: both low halves, then both high ones, so that few roundings are
+                        // at full size; group 16: low and high of one fragment at a time
+                        const bool g32 = W::kGroup == 32u;
+                        const uint32_t h = g32 ? k & 1u : k / 2u, p = g32 ? k < 2u : !(k & 1u);
+                        const f16x8 f = afrag(buf, m, p, h);
 #pragma unroll
-                            for (uint32_t r = 0; r < 16; ++r) acc[m][0][r] = __builtin_fmaf(ds[0][h], P[r], acc[m][0][r]);
+                        for (uint32_t i = 0; i < 2; ++i)
+                            P[i] = mfma(f, b[i][h], (g32 ? k : k & 1u) == 0u ? f32x16{} : P[i]);
+                        if (k == 3u || (!g32 && k == 1u)) {
 #pragma unroll
-                            for (uint32_t r = 0; r < 16; ++r) acc[m][1][r] = __builtin_fmaf(ds[1][h], Q[r], acc[m][1][r]);
+                            for (uint32_t i = 0; i < 2; ++i)
+#pragma unroll
+                                for (uint32_t r = 0; r < 16; ++r)
+                                    acc[m][i][r] = __builtin_fmaf(ds[i][h], P[i][r], acc[m][i][r]);
                         }
                     }
                 }
@@ -656,6 +670,9 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
             load_act((j + 1u) % NS, s + 1u + NS);
             if (j == 4u) store_sums(sbuf ^ 1u);
             __syncthreads();
+            // Q4_K: keeps the next step's decoding behind this one's products (without it 6
+            // registers spill; Q5_K has none to spare either way and is 4% slower with it)
+            if constexpr (kHalves && T == T_Q4_K) __builtin_amdgcn_sched_barrier(0);
         }
     }
 

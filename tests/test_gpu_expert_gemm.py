@@ -82,6 +82,57 @@ def test_zero_and_spread_block_scales(hip, port, gtype):
     check(hip, port, layer, x, who, range(0, who.size, 29))
 
 
+def centred_matrix(gtype, rows, cols, gen):
+    """Q4_K or Q5_K rows whose weights lie around zero, as trained ones do: uniform
+    quants, 6-bit scales 20 to 63, the mins the same numbers, dmin the mid quant times d."""
+    b = gen.integers(0, 256, (rows * cols // 256, S.BLOCK_BYTES[gtype]), dtype=np.uint8)
+    q, mid = (4.6, 7.5) if gtype == S.Q4_K else (9.2, 15.5)
+    d = (0.02 / (q * 42.0) * gen.uniform(0.75, 1.25, len(b))).astype(np.float16)
+    b[:, 0:2] = d.view(np.uint8).reshape(-1, 2)
+    b[:, 2:4] = (d.astype(np.float32) * mid).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    sc = gen.integers(20, 64, (len(b), 8), dtype=np.uint8)
+    b[:, 4:8] = b[:, 8:12] = (sc[:, :4] & 63) | ((sc[:, 4:] >> 4) << 6)
+    b[:, 12:16] = (sc[:, 4:] & 15) | ((sc[:, 4:] & 15) << 4)
+    return b.reshape(-1)
+
+
+def float64_error(hip, port, gtype, hidden, ffn, tokens, experts=4):
+    """2-norm of the prefill's difference from float64 over the result's."""
+    g = S.rng(980 + hidden + tokens)
+    layer = S.moe_layer(seed=981, hidden=hidden, experts=experts, ffn=ffn, top_k=1, gate_type=gtype,
+                        up_type=gtype, down_type=gtype)
+    layer.gate, layer.up = (centred_matrix(gtype, experts * ffn, hidden, g) for _ in range(2))
+    layer.down = centred_matrix(gtype, experts * hidden, ffn, g)
+    x = S.normal_f32(g, tokens * hidden).reshape(tokens, hidden)
+    h = hip.upload_moe_layer(layer)
+    y, ids, _ = hip.moe_prefill(h, x)
+    h.release()
+
+    def w(data, e, rows, cols):
+        n = len(data) // experts
+        f = port.dequantize_row(gtype, data[e * n:(e + 1) * n], rows * cols)
+        return f.astype(np.float64).reshape(rows, cols)
+
+    want = np.zeros((tokens, hidden))
+    for e in range(experts):
+        t = ids[:, 0] == e
+        xe = x[t].astype(np.float64)
+        gate, up = xe @ w(layer.gate, e, ffn, hidden).T, xe @ w(layer.up, e, ffn, hidden).T
+        want[t] = (gate / (1.0 + np.exp(-gate)) * up) @ w(layer.down, e, hidden, ffn).T
+    return float(np.linalg.norm(y - want) / np.linalg.norm(want))
+
+
+@pytest.mark.parametrize("tokens", (20, 300))  # 32-row tiles, 64-row tiles
+@pytest.mark.parametrize("hidden,bound", ((512, 2.87e-7), (1024, 3.35e-7), (2048, 4.1e-7)))
+def test_q5_k_error_against_float64(hip, port, hidden, bound, tokens):
+    """The bounds are what GEMMs on three exact bf16 parts of x, with one FP32 sum per
+    32 values, have on these inputs; two fp16 halves must not be further off (2.7e-7,
+    3.1e-7 and 3.5e-7; one sum of both halves over 256 values: 3.2e-7, 3.4e-7, 3.8e-7)."""
+    err = float64_error(hip, port, S.Q5_K, hidden, 512, tokens)
+    print(f"Q5_K hidden {hidden} tokens {tokens}: {err:.3g}")
+    assert err <= bound
+
+
 def test_activation_range(hip, port):
     """Rows scaled by 1e-12 to 1e12, and values far below their row's maximum."""
     layer, x, who = grouped_layer(S.Q4_K, S.Q6_K, 970)
