@@ -411,6 +411,7 @@ struct GemmShared {
     uint8_t xs[2][kGemmTileM * 32u];        // group sums of two superblocks: 8 hi, 8 lo
     uint32_t arow[kGemmTileM], oslot[kGemmTileM];
     float scale[kGemmTileM];
+    uint32_t far;  // down: some row's chunk scales are far apart
 };
 
 // Maximum of |v| over each 32-lane half, in all its lanes (as unsigned bits, whose
@@ -426,12 +427,14 @@ __device__ __forceinline__ float half_wave_max(float v) {
     return __uint_as_float(max(s[0], s[1]));
 }
 
-// MT x 32 assignments of a tile.  DUAL: gate and up rows n0 .. n0 + 127 over x,
-// SwiGLU, activations split for the down GEMM; otherwise down rows n0 .. n0 + 255
-// over the activations, each output row to its (token, route) slot.
-template <int T, bool UNITS, bool DUAL, int MT>
+// MT x 32 assignments of a tile, from its row row0.  DUAL: gate and up rows n0 .. n0 + 127
+// over x, SwiGLU, activations split for the down GEMM; otherwise down rows n0 .. n0 + 255
+// over the activations, each output row to its (token, route) slot.  FAR: some chunk's
+// scale lies more than 2^24 below its row's, and the halves come down in two steps.
+// (Two steps in every tile leave Q6_K's down no registers: 4096 tokens 1106 -> 1342 us.)
+template <int T, bool UNITS, bool DUAL, int MT, bool FAR = false>
 __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef& tr, uint32_t n0,
-                                          GemmShared& sh) {
+                                          GemmShared& sh, uint32_t row0 = 0u) {
     using W = WTraits<T, UNITS>;
     const MoeDecodeArgs& L = a.layer;
     const uint32_t kdim = DUAL ? L.hidden : L.ffn, ndim = DUAL ? L.ffn : L.hidden;
@@ -476,16 +479,16 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const uint32_t row = pr + 32u * i;
-        asrc[i] = parts + static_cast<uint64_t>(sh.arow[row]) * kdim * 2u + pc * 8u;
+        asrc[i] = parts + static_cast<uint64_t>(sh.arow[row0 + row]) * kdim * 2u + pc * 8u;
         adst[i] = row * kStageRow + ((pc ^ (row & 7u)) * 16u);
-        csrc[i] = DUAL ? nullptr : a.act_scale + static_cast<uint64_t>(sh.arow[row]) * nst;
-        cinv[i] = DUAL ? 0.0f : 1.0f / sh.scale[row];
+        csrc[i] = DUAL ? nullptr : a.act_scale + static_cast<uint64_t>(sh.arow[row0 + row]) * nst;
+        cinv[i] = DUAL ? 0.0f : 1.0f / sh.scale[row0 + row];
     }
     // register sets of stages in flight: with one row block there is room for eight,
     // which small batches need, where little else hides the loads' latency (77
     // tokens, 64 experts: gate/up 45 -> 42 us; 512 tokens 119 -> 117); Q5_K's down has
     // room for four
-    constexpr uint32_t NS = MT == 1 ? (T == T_Q5_K && !DUAL ? 4u : 8u) : 2u;
+    constexpr uint32_t NS = MT == 2 || FAR ? 2u : T == T_Q5_K && !DUAL ? 4u : 8u;
     u32x4_t av[NS][MT];
     float ac[NS][MT];
     const uint32_t last = 8u * nsb - 1u;
@@ -502,10 +505,20 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         for (int i = 0; i < MT; ++i) {
             u32x4_t v = av[set][i];
             if constexpr (!DUAL) {  // from the chunk's scale to the row's (a power of two, at most 1)
-                const _Float16 f = static_cast<_Float16>(ac[set][i] * cinv[i]);
-                const f16x2 ff = {f, f};
+                const float r = ac[set][i] * cinv[i];
+                if constexpr (FAR) {  // FP16 ends at 2^-24: the rest as a second factor
+                    const bool far = r < 0x1p-24f;
+                    const f16x2 g = __builtin_bit_cast(f16x2, far ? 0x00010001u : 0x3c003c00u);  // 2^-24, 1
+                    const _Float16 f = static_cast<_Float16>(far ? r * 0x1p24f : r);
+                    const f16x2 ff = {f, f};
 #pragma unroll
-                for (int k = 0; k < 4; ++k) v[k] = pk_mul_f16(v[k], ff);
+                    for (int k = 0; k < 4; ++k) v[k] = pk_mul_f16(pk_mul_f16(v[k], ff), g);
+                } else {
+                    const _Float16 f = static_cast<_Float16>(r);
+                    const f16x2 ff = {f, f};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[k] = pk_mul_f16(v[k], ff);
+                }
             }
             *reinterpret_cast<u32x4_t*>(sh.st[buf] + adst[i]) = v;
         }
@@ -517,8 +530,8 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     // block, 340 with two; none without the branch).  kUnits, with no FMA per step,
     // fits better with it (208 registers against 256 and 25 spilled).
     const uint32_t dr = tid / 4u, sr = dr < 32u * MT ? dr : 0u, sg = 2u * (tid % 4u);
-    const float* ssrc = W::kMins ? sums + static_cast<uint64_t>(sh.arow[sr]) * nst + sg : nullptr;
-    const float sinv = W::kMins ? (W::kMinsF32 ? 1.0f : 0x1p-5f) / sh.scale[sr] : 0.0f;
+    const float* ssrc = W::kMins ? sums + static_cast<uint64_t>(sh.arow[row0 + sr]) * nst + sg : nullptr;
+    const float sinv = W::kMins ? (W::kMinsF32 ? 1.0f : 0x1p-5f) / sh.scale[row0 + sr] : 0.0f;
     float2 sv = make_float2(0.0f, 0.0f);
     auto load_sums = [&](uint32_t sb) {
         if constexpr (W::kMins) sv = *reinterpret_cast<const float2*>(ssrc + 8u * (sb < nsb ? sb : nsb - 1u));
@@ -697,7 +710,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         for (int m = 0; m < MT; ++m) {
 #pragma unroll
             for (uint32_t r = 0; r < 16; ++r) {
-                const uint32_t row = 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
+                const uint32_t row = row0 + 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
                 const float s = sh.scale[row];
                 const float g = acc[m][0][r] * (u0 * s), u = acc[m][1][r] * (u1 * s);
                 const float v = (g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))) * u;
@@ -725,7 +738,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (uint32_t r = 0; r < 16; ++r) {
-                const uint32_t row = 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
+                const uint32_t row = row0 + 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
                 if (row < tr.rows) {
                     const float s = sh.scale[row];
                     float* o = out + static_cast<uint64_t>(sh.oslot[row]) * ndim + n0 + wave * 32u + ln;
@@ -756,16 +769,38 @@ __global__ __launch_bounds__(256, 2) void k_expert_gemm(MoePrefillArgs a) {
         if constexpr (DUAL) sh.scale[tid] = a.x_scale[row];
     }
     if constexpr (!DUAL) {  // a row's scale: the largest of its chunks'
+        if (tid == 0u) sh.far = 0u;
         __syncthreads();
         const uint32_t row = tid / 4u, nch = L.ffn / 32u;
         const float* cs = a.act_scale + static_cast<uint64_t>(sh.arow[row]) * nch;
+        // the least scale of a chunk that is not zero, as bits past kZeroScale's (a zero
+        // chunk's wrap around)
+        const uint32_t past = __float_as_uint(kZeroScale) + 1u;
         float m = 0.0f;
-        for (uint32_t c = tid % 4u; c < nch; c += 4u) m = fmaxf(m, cs[c]);
+        uint32_t least = ~0u;
+        for (uint32_t c = tid % 4u; c < nch; c += 4u) {
+            const float s = cs[c];
+            m = fmaxf(m, s);
+            least = min(least, __float_as_uint(s) - past);
+        }
         m = fmaxf(m, dpp<0xb1>(m));
         m = fmaxf(m, dpp<0x4e>(m));
+        // (below 2^-84 what has the zero scale may not be nothing to the row; at 2^-102 and
+        // below no scale lies 2^24 under it)
+        if (m > 0x1p-102f && (m < 0x1p-84f || least < __float_as_uint(m * 0x1p-24f) - past)) sh.far = 1u;
         if (tid % 4u == 0u) sh.scale[row] = m;
     }
     __syncthreads();
+    if constexpr (!DUAL) {
+        if (__builtin_amdgcn_readfirstlane(sh.far)) {  // rare: outliers in the activations
+#pragma nounroll
+            for (uint32_t row0 = 0; row0 < tr.rows; row0 += 32u) {
+                if (row0) __syncthreads();  // the rows before are past their last read
+                gemm_tile<T, UNITS, false, 1, true>(a, tr, yb * nblk, sh, row0);
+            }
+            return;
+        }
+    }
     if (tr.rows > 32u) {
         gemm_tile<T, UNITS, DUAL, 2>(a, tr, yb * nblk, sh);
     } else {

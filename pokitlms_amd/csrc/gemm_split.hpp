@@ -7,7 +7,9 @@
 // significant bits of every value above 2^-15 of the row's maximum and an
 // absolute error of 2^-39 of that maximum below (fp16 subnormals, which the
 // MFMA reads exactly): FP32's own rounding, at two MFMAs per product where
-// three bf16 parts take three.
+// three bf16 parts take three.  Chunks are brought to their row's scale by a power
+// of two when the GEMM loads them, which rounds their halves to the same absolute
+// step: 2^-38 of the row's maximum at most.
 //
 // Rows are stored as [row][32-value stage][hi, lo][32], so one stage of a row
 // is one 128-byte line; inside each run of 8 values the order is 0, 2, 1, 3, 4,
@@ -37,6 +39,8 @@ __device__ __forceinline__ void split_scale(float m, float& s, float& inv) {
     s = __uint_as_float((e - 14u) << 23);
     inv = __uint_as_float((268u - e) << 23);
 }
+
+constexpr float kZeroScale = 0x1p-126f;  // the scale of a zero row or chunk (or one below 2^-112)
 
 // Two scaled values as (hi, hi) and (lo, lo) dwords.
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {

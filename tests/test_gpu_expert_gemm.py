@@ -141,3 +141,46 @@ def test_activation_range(hip, port):
     x *= scale[:, None]
     layer.router *= np.float32(1e-3)
     check(hip, port, layer, x, who, range(0, who.size, 2))
+
+
+@pytest.mark.parametrize("down_type", QUANT, ids=lambda t: S.TYPE_NAMES[t])
+@pytest.mark.parametrize("ratio", (22, 24, 25, 26, 28))
+def test_chunks_far_below_their_row(hip, port, down_type, ratio):
+    """Activations whose first 32 values are 2^ratio times the others (from Q8_0 up rows
+    of such scales) and whose down weights there are zero: what is left comes from the
+    small chunks alone.  Each of a value's two halves is rounded to 2^-39 of the row's
+    maximum, together 2^(ratio - 38) of the small chunks' maximum; a value is about half
+    of that, and quants and mins summed apart take both: 2^(ratio - 36).  One expert has
+    20 rows, one 50."""
+    hidden, ffn = 512, 256
+    layer = S.moe_layer(seed=990, hidden=hidden, experts=2, ffn=ffn, top_k=1, gate_type=S.Q8_0,
+                        up_type=S.Q8_0, down_type=down_type)
+    layer.router = np.zeros((2, hidden), np.float32)
+    layer.router[:, 2:4] = np.eye(2, dtype=np.float32)
+    gate = np.zeros((2 * ffn, hidden // 32, 34), np.uint8)
+    gate[:, 0, 0:2] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)
+    gate[:, 0, 2] = 1  # g = x[0]
+    layer.gate = gate.reshape(-1)
+    up = layer.up.reshape(2, ffn, hidden // 32, 34)
+    for rows, d in ((up[:, :32], 2.0 ** 9), (up[:, 32:], 2.0 ** (9 - ratio))):
+        rows[..., 0:2] = np.frombuffer(np.float16(d).tobytes(), np.uint8)
+    down = layer.down.reshape(2 * hidden, -1, S.BLOCK_BYTES[down_type])[:, 0]  # each row's first block
+    if down_type in (S.Q4_K, S.Q5_K):
+        down[:, 4] &= 0xC0  # scale and min of the first group
+        down[:, 8] &= 0xC0
+    elif down_type == S.Q6_K:
+        down[:, 192:194] = 0
+    else:
+        down[:, 0:4 if down_type == S.Q4_1 else 2] = 0
+    who = np.repeat((0, 1), (20, 50))
+    x = S.normal_f32(S.rng(991), who.size * hidden).reshape(who.size, hidden)
+    x[:, 0] = 6.0
+    x[:, 2:4] = 0.0
+    x[np.arange(who.size), 2 + who] = 30.0
+    h = hip.upload_moe_layer(layer)
+    y, ids, _ = hip.moe_prefill(h, x)
+    h.release()
+    assert np.array_equal(ids[:, 0], who)
+    blk = port.moe(layer)
+    for t in range(0, who.size, 3):
+        assert normwise_rel(y[t], blk.forward(x[t])[0]) <= max(TOL, 2.0 ** (ratio - 36)), (t, who[t])
