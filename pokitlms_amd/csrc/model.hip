@@ -383,7 +383,9 @@ __global__ __launch_bounds__(256) void k_argmax(ModelArgs a, uint32_t parts) {
     if (tid == 0) {
         for (uint32_t w = 1; w < 4; ++w) argmax_merge(bv[0], bi[0], bv[w], bi[w]);
         const uint32_t pos = a.state[0];
-        if (pos + 1u >= a.state[1]) a.tokens[pos + 1u] = bi[0];  // past the prompt: generated
+        // past the prompt: generated.  With every logit NaN there is no maximum (the
+        // chunks have flagged it); the steps already enqueued read row 0 then.
+        if (pos + 1u >= a.state[1]) a.tokens[pos + 1u] = bi[0] < a.vocab ? bi[0] : 0u;
         a.state[0] = pos + 1u;
     }
 }

@@ -253,3 +253,20 @@ def test_embedding_row_types(hip, port, embd_type):
     say("embedding", S.TYPE_NAMES[embd_type], "tokens", t0)
     assert np.array_equal(t0, t1)
     assert np.array_equal(l0.view(np.uint32), l1.view(np.uint32))
+
+
+@pytest.mark.parametrize("reference_order", (True, False), ids=("reference", "fast"))
+def test_nan_logits_are_an_error(hip, reference_order):
+    """Every logit NaN: no maximum, so the steps already enqueued behind it must still
+    read a token of the vocabulary; the call reports the error."""
+    from pokitlms_amd.backend import HipError
+    from pokitlms_amd.model import Qwen3MoeModel
+    m = SM.Qwen3MoeShape(layers=1, hidden=512, heads=8, kv_heads=4, head_dim=64, experts=16, top_k=4,
+                         ffn=256, vocab=2048)
+    weights = Qwen3MoeModel.synthetic_weights(hip, m, 31)
+    weights["output_norm.weight"].release()
+    weights["output_norm.weight"] = hip.upload(S.F32, m.hidden, 1, np.full(m.hidden, np.nan, np.float32))
+    with Qwen3MoeModel(hip, m, weights, reference_order) as model:
+        for n in (1, 20):
+            with pytest.raises(HipError, match="non-finite"):
+                model.generate(SM.prompt_tokens(5, n, m.vocab), 4)

@@ -95,3 +95,22 @@ def test_formats(hip, gtype):
                 got, _, _ = model.generate(seq[:n], 4)
                 assert np.array_equal(got, seq[n:n + 4]), (start, n)
     assert len(seen) >= 3  # sequences worth comparing
+
+
+@pytest.mark.parametrize("n", (1, 4, 40))
+def test_non_finite_prompt_is_an_error(hip, n):
+    """Non-finite router logits in a token step, in a chunk that takes its routes one by
+    one (3 positions, 12 routes) and in one that groups them: every route falls to
+    expert 0 and the call reports the error."""
+    from pokitlms_amd.backend import HipError
+    from pokitlms_amd.model import Qwen3MoeModel
+    m = shape()
+    weights = Qwen3MoeModel.synthetic_weights(hip, m, 31)
+    bad = np.ones(m.hidden, np.float32)
+    bad[7] = np.inf
+    weights["blk.0.ffn_norm.weight"].release()
+    weights["blk.0.ffn_norm.weight"] = hip.upload(S.F32, m.hidden, 1, bad)
+    with Qwen3MoeModel(hip, m, weights) as model:
+        for _ in range(2):
+            with pytest.raises(HipError, match="non-finite"):
+                model.generate(SM.prompt_tokens(3, n, m.vocab), 3)
