@@ -134,11 +134,14 @@ def test_q5_k_error_against_float64(hip, port, hidden, bound, tokens):
 
 
 def test_activation_range(hip, port):
-    """Rows scaled by 1e-12 to 1e12, and values far below their row's maximum."""
+    """Rows scaled by 1e-12 to 1e12, and values down to 2^-27 of their row's maximum; a
+    zero row, and one so small that its scale is the smallest there is."""
     layer, x, who = grouped_layer(S.Q4_K, S.Q6_K, 970)
     x[:, 64:] *= np.float32(2.0) ** -np.arange(0, 28).repeat(16).astype(np.float32)
-    scale = np.float32(10.0) ** (np.arange(who.size) % 13 - 6).astype(np.float32)
-    x *= scale[:, None]
+    x *= (np.float32(10.0) ** (np.arange(who.size) % 25 - 12).astype(np.float32))[:, None]
+    x[0] = 0.0  # every logit equal: the first expert
+    who[0] = 0
+    x[2] = x[2] / np.abs(x[2]).max() * np.float32(1e-35)
     layer.router *= np.float32(1e-3)
     check(hip, port, layer, x, who, range(0, who.size, 2))
 

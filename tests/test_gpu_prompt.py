@@ -4,8 +4,9 @@ The reference-order model is the CPU's bits (tests/test_gpu_model.py); the fast
 mode is within FP32 reassociation of it, which two layers carry to about 5e-5
 normwise in the logits, and to 1e-3 where a rounding decides a router near-tie
 (the bound tests/test_gpu_model.py holds every depth to).  Prompt lengths on both
-sides of the shortest batch (5 positions, then the last token as a step), of the
-32- and 64-row tiles, of one chunk, and of the KV window.
+sides of the shortest batch (5 positions, then the last token as a step), of a
+32-row tile's end, of one chunk, and of the KV window; a model wide enough for the
+projections' 64-row tiles; every attention format the batch takes.
 """
 import numpy as np
 import pytest
@@ -55,6 +56,42 @@ def test_prompt_formats(hip, kw):
     q wider than the hidden state."""
     for n in (40, 200):
         compare(hip, shape(**kw), n)
+
+
+@pytest.mark.parametrize("n", (449, 450, 498, 513))
+def test_prompt_wide_projections(hip, n):
+    """q, k and v of 9216 rows: 449 positions and more make too many 32-row tiles for the
+    chip, so the projections take 64-row ones (the last one short, or whole at 512)."""
+    compare(hip, SM.Qwen3MoeShape(layers=1, hidden=512, heads=64, kv_heads=4, head_dim=128, experts=16,
+                                  top_k=4, ffn=256, vocab=2048), n)
+
+
+@pytest.mark.parametrize("gtype", (S.Q4_0, S.Q4_1, S.Q8_0), ids=lambda t: S.TYPE_NAMES[t])
+def test_prompt_attention_formats(hip, gtype):
+    """The projections in the formats the synthetic model has no recipe for."""
+    from pokitlms_amd.model import Qwen3MoeModel
+    m = shape()
+    out = []
+    for reference_order in (True, False):
+        weights = Qwen3MoeModel.synthetic_weights(hip, m, 31)
+        gen = S.rng(70 + gtype)
+        for layer in range(m.layers):
+            for name, inn, rows in (("attn_q", 512, 512), ("attn_k", 512, 256), ("attn_v", 512, 256),
+                                    ("attn_output", 512, 512)):
+                data = S.quant_matrix(gtype, rows, inn, gen)
+                blocks = data.reshape(-1, S.BLOCK_BYTES[gtype])
+                flip = gen.integers(0, 2, len(blocks), dtype=np.uint8) << 7
+                for off in S.SCALE_OFFSETS[gtype]:  # half the blocks negated: weights around zero
+                    blocks[:, off + 1] ^= flip
+                key = f"blk.{layer}.{name}.weight"
+                weights[key].release()
+                weights[key] = hip.upload(gtype, inn, rows, data)
+        with Qwen3MoeModel(hip, m, weights, reference_order) as model:
+            out.append([model.generate(SM.prompt_tokens(n, n, m.vocab), 4, want_logits=True)
+                        for n in (8, 40, 200)])
+    for (want, wl, _), (got, gl, _) in zip(*out):
+        assert normwise_rel(gl, wl) <= 1e-3
+        assert np.array_equal(got, want)
 
 
 def test_prompt_narrow_kv_takes_steps(hip):
