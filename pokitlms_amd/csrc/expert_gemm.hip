@@ -75,10 +75,11 @@ __device__ __forceinline__ uint32_t pk_mul_f16(uint32_t a, f16x2 b) {
 //    term (16 d sc - dmin m) times the FP32 group sums on FP32 MFMA.  With two row
 //    blocks each step's sum goes into the accumulator by an FMA with d, as the other
 //    formats' do; with one there are registers for sums over the superblock, the high
-//    and the low halves' apart (kHalves), which is a chain less to wait for.  A single
-//    sum of both over the superblock was 20% further from float64 at hidden 512 (Q5_K
-//    3.5e-7 against 2.9e-7; 1024: 3.7e-7 against 3.2e-7, 2048: 4.5e-7 against 4.3e-7) and
-//    spilled 13 to 23 registers (2048 tokens 735 -> 701 us without, 77 tokens level).
+//    and the low halves' apart (kHalves): the FMA per step would wait for its products
+//    there (77 tokens, hidden 1024, prefill 69.9 -> 74.8 us).  A single sum of both over
+//    the superblock was 20% further from float64 at hidden 512 (Q5_K 3.5e-7 against
+//    2.9e-7; 1024: 3.7e-7 against 3.2e-7, 2048: 4.5e-7 against 4.3e-7) and spilled 13 to 23
+//    registers (2048 tokens 735 -> 701 us without, 77 tokens 68.7 -> 69.4).
 //    As kUnits, Q5_K had 6.1e-7 (the larger quants leave more to cancel against the
 //    mins), and Q4_K projections at 8.7e-7 put the whole model's logits 15% further from
 //    float64, as fewer FP16 roundings of k then agree; the MoE block's gate/up keeps the
@@ -625,9 +626,11 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
                         acc[m][1] = mfma(hi, b[1][h], acc[m][1]);
                     }
             } else if constexpr (kHalves) {
+                // low and high of one fragment, then of the other; in the superblock's last step
+                // both low ones first, whose sums go into the accumulator while the high ones end
 #pragma unroll
-                for (uint32_t k = 0; k < 4; ++k) {  // hi and lo of the first fragment, then of the second
-                    const uint32_t h = k / 2u, p = k & 1u;
+                for (uint32_t k = 0; k < 4; ++k) {
+                    const uint32_t h = j == 7u ? k & 1u : k / 2u, p = j == 7u ? k < 2u : !(k & 1u);
                     const f16x8 f = afrag(buf, 0u, p, h);
 #pragma unroll
                     for (uint32_t i = 0; i < 2; ++i)
@@ -635,10 +638,12 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
                 }
                 if (j == 7u) {
 #pragma unroll
-                    for (uint32_t i = 0; i < 2; ++i)
+                    for (uint32_t q = 0; q < 2; ++q)
 #pragma unroll
-                        for (uint32_t r = 0; r < 16; ++r)
-                            acc[0][i][r] = __builtin_fmaf(hd[i].d, half[i][0][r] + half[i][1][r], acc[0][i][r]);
+                        for (uint32_t i = 0; i < 2; ++i)
+#pragma unroll
+                            for (uint32_t r = 0; r < 16; ++r)
+                                acc[0][i][r] = __builtin_fmaf(hd[i].d, half[i][1u - q][r], acc[0][i][r]);
                 }
             } else {
 #pragma unroll
