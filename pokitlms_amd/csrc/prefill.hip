@@ -67,7 +67,8 @@ struct RouterSums {
 // Lane (i, j) of a wave takes tokens TT i .. and rows TE j ..: 8 TT tokens x 8 TE
 // rows per workgroup.  2 x 4 where that makes two workgroups per CU, else 1 x 2
 // (a wave's chain is a quarter as long: 512 tokens 33 -> 21 us, 77 tokens x 64
-// rows of 1024 17 -> 6 us).
+// rows of 1024 17 -> 6 us).  The first form spills seven registers of addresses, which
+// a stage of 768 vector instructions reads back once; 32-bit offsets spill as many.
 template <uint32_t TT, uint32_t TE>
 __global__ __launch_bounds__(64 * kRtWaves, 4) void k_router_batch(MoePrefillArgs a) {
     constexpr uint32_t T = 8u * TT, R = 8u * TE, NL = TT + TE;
