@@ -430,14 +430,14 @@ __device__ __forceinline__ float half_wave_max(float v) {
     return __uint_as_float(max(s[0], s[1]));
 }
 
-// MT x 32 assignments of a tile, from its row row0.  DUAL: gate and up rows n0 .. n0 + 127
-// over x, SwiGLU, activations split for the down GEMM; otherwise down rows n0 .. n0 + 255
+// MT x 32 assignments of a tile.  DUAL: gate and up rows n0 .. n0 + 127 over x, SwiGLU, activations split for the down GEMM; otherwise down rows n0 .. n0 + 255
 // over the activations, each output row to its (token, route) slot.  FAR: some chunk's
-// scale lies more than 2^24 below its row's, and the halves come down in two steps.
-// (Two steps in every tile leave Q6_K's down no registers: 4096 tokens 1106 -> 1342 us.)
+// scale lies more than 2^24 below its row's, and the halves come down in two steps
+// (in every tile 0.5 to 2% slower, Q6_K 20%; in tiles that need it, one row block at a
+// time, a 512-token batch with such rows 4 us slower, 110 -> 118 us for down).
 template <int T, bool UNITS, bool DUAL, int MT, bool FAR = false>
 __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef& tr, uint32_t n0,
-                                          GemmShared& sh, uint32_t row0 = 0u) {
+                                          GemmShared& sh) {
     using W = WTraits<T, UNITS>;
     const MoeDecodeArgs& L = a.layer;
     const uint32_t kdim = DUAL ? L.hidden : L.ffn, ndim = DUAL ? L.ffn : L.hidden;
@@ -482,10 +482,10 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const uint32_t row = pr + 32u * i;
-        asrc[i] = parts + static_cast<uint64_t>(sh.arow[row0 + row]) * kdim * 2u + pc * 8u;
+        asrc[i] = parts + static_cast<uint64_t>(sh.arow[row]) * kdim * 2u + pc * 8u;
         adst[i] = row * kStageRow + ((pc ^ (row & 7u)) * 16u);
-        csrc[i] = DUAL ? nullptr : a.act_scale + static_cast<uint64_t>(sh.arow[row0 + row]) * nst;
-        cinv[i] = DUAL ? 0.0f : 1.0f / sh.scale[row0 + row];
+        csrc[i] = DUAL ? nullptr : a.act_scale + static_cast<uint64_t>(sh.arow[row]) * nst;
+        cinv[i] = DUAL ? 0.0f : 1.0f / sh.scale[row];
     }
     // register sets of stages in flight: with one row block there is room for eight,
     // which small batches need, where little else hides the loads' latency (77
@@ -533,8 +533,8 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     // block, 340 with two; none without the branch).  kUnits, with no FMA per step,
     // fits better with it (208 registers against 256 and 25 spilled).
     const uint32_t dr = tid / 4u, sr = dr < 32u * MT ? dr : 0u, sg = 2u * (tid % 4u);
-    const float* ssrc = W::kMins ? sums + static_cast<uint64_t>(sh.arow[row0 + sr]) * nst + sg : nullptr;
-    const float sinv = W::kMins ? (W::kMinsF32 ? 1.0f : 0x1p-5f) / sh.scale[row0 + sr] : 0.0f;
+    const float* ssrc = W::kMins ? sums + static_cast<uint64_t>(sh.arow[sr]) * nst + sg : nullptr;
+    const float sinv = W::kMins ? (W::kMinsF32 ? 1.0f : 0x1p-5f) / sh.scale[sr] : 0.0f;
     float2 sv = make_float2(0.0f, 0.0f);
     auto load_sums = [&](uint32_t sb) {
         if constexpr (W::kMins) sv = *reinterpret_cast<const float2*>(ssrc + 8u * (sb < nsb ? sb : nsb - 1u));
@@ -717,7 +717,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         for (int m = 0; m < MT; ++m) {
 #pragma unroll
             for (uint32_t r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
+                const uint32_t row = 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
                 const float s = sh.scale[row];
                 const float g = acc[m][0][r] * (u0 * s), u = acc[m][1][r] * (u1 * s);
                 const float v = (g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))) * u;
@@ -745,7 +745,7 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (uint32_t r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
+                const uint32_t row = 32u * m + (r / 4u) * 8u + kq * 4u + (r % 4u);
                 if (row < tr.rows) {
                     const float s = sh.scale[row];
                     float* o = out + static_cast<uint64_t>(sh.oslot[row]) * ndim + n0 + wave * 32u + ln;
@@ -799,12 +799,9 @@ __global__ __launch_bounds__(256, 2) void k_expert_gemm(MoePrefillArgs a) {
     }
     __syncthreads();
     if constexpr (!DUAL) {
-        if (__builtin_amdgcn_readfirstlane(sh.far)) {  // rare: outliers in the activations
-#pragma nounroll
-            for (uint32_t row0 = 0; row0 < tr.rows; row0 += 32u) {
-                if (row0) __syncthreads();  // the rows before are past their last read
-                gemm_tile<T, UNITS, false, 1, true>(a, tr, yb * nblk, sh, row0);
-            }
+        if (__builtin_amdgcn_readfirstlane(sh.far)) {  // outliers in the activations
+            if (tr.rows > 32u) gemm_tile<T, UNITS, false, 2, true>(a, tr, yb * nblk, sh);
+            else gemm_tile<T, UNITS, false, 1, true>(a, tr, yb * nblk, sh);
             return;
         }
     }
