@@ -74,18 +74,20 @@ __device__ __forceinline__ uint32_t pk_mul_f16(uint32_t a, f16x2 b) {
 //  * Q5_K, and Q4_K in the prompt's projections: q - 16 (q - 8), the rest of the mins'
 //    term (16 d sc - dmin m) times the FP32 group sums on FP32 MFMA.  With two row
 //    blocks each step's sum goes into the accumulator by an FMA with d, as the other
-//    formats' do; with one there are registers for sums over the superblock, the high
-//    and the low halves' apart (kHalves): the FMA per step would wait for its products
-//    there (77 tokens, hidden 1024, prefill 69.9 -> 74.8 us).  A single sum of both over
-//    the superblock was 20% further from float64 at hidden 512 (Q5_K 3.5e-7 against
-//    2.9e-7; 1024: 3.7e-7 against 3.2e-7, 2048: 4.5e-7 against 4.3e-7) and spilled 13 to 23
-//    registers (2048 tokens 735 -> 701 us without, 77 tokens 68.7 -> 69.4).
+//    formats' do; with one there are registers for sums over the superblock (kSums),
+//    as the FMA per step would wait for its products there (77 tokens, hidden 1024,
+//    prefill 69.9 -> 74.8 us).  Q5_K keeps the high and the low halves' apart: a single sum
+//    was 20% further from float64 at hidden 512 (3.5e-7 against 2.9e-7; 1024: 3.7e-7
+//    against 3.2e-7, 2048: 4.5e-7 against 4.3e-7), and with two row blocks spilled 13 to
+//    23 registers (2048 tokens 735 -> 701 us without, 77 tokens 68.7 -> 69.4).  Only at
+//    hidden 4096 and two row blocks, where the FMAs are many, was it closer (4.7e-7
+//    against 5.0e-7; exact bf16 parts 5.6e-7); two steps to an FMA spill again.  Q4_K
+//    projections keep the single sum (4.0e-7): the model's logits are as far from
+//    float64 as with a token step per position (0.995 +- 0.014 of that over 294 prompts).
 //    As kUnits, Q5_K had 6.1e-7 (the larger quants leave more to cancel against the
 //    mins), and Q4_K projections at 8.7e-7 put the whole model's logits 15% further from
 //    float64, as fewer FP16 roundings of k then agree; the MoE block's gate/up keeps the
-//    units, 472 against 557 us at 4096 tokens: in the prompt they change nothing of the
-//    logits' error, which is the projections' (over 294 prompts of 1 to 4 layers it is
-//    0.92 of that of one token step per position).
+//    units, 472 against 557 us at 4096 tokens, and does not show in the logits.
 //
 // The others: quants as exact fp16 integers around zero (1024 + q by or-ing the
 // exponent in, minus 1024 and the offset), and per scale group (32 values;
@@ -430,11 +432,11 @@ __device__ __forceinline__ float half_wave_max(float v) {
     return __uint_as_float(max(s[0], s[1]));
 }
 
-// MT x 32 assignments of a tile.  DUAL: gate and up rows n0 .. n0 + 127 over x, SwiGLU, activations split for the down GEMM; otherwise down rows n0 .. n0 + 255
-// over the activations, each output row to its (token, route) slot.  FAR: some chunk's
-// scale lies more than 2^24 below its row's, and the halves come down in two steps
-// (in every tile 0.5 to 2% slower, Q6_K 20%; in tiles that need it, one row block at a
-// time, a 512-token batch with such rows 4 us slower, 110 -> 118 us for down).
+// MT x 32 assignments of a tile.  DUAL: gate and up rows n0 .. n0 + 127 over x, SwiGLU,
+// activations split for the down GEMM; otherwise down rows n0 .. n0 + 255 over the
+// activations, each output row to its (token, route) slot.  FAR: some chunk's scale
+// lies more than 2^24 below its row's, and the halves come down in two steps (which in
+// every tile would cost 0.5 to 2%).
 template <int T, bool UNITS, bool DUAL, int MT, bool FAR = false>
 __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef& tr, uint32_t n0,
                                           GemmShared& sh) {
@@ -571,8 +573,9 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
     load_act(0u, 8u * sb0 + NS);
     __syncthreads();
 
-    f32x16 acc[MT][2], half[2][2];  // half: kHalves, the superblock's sums of the high and low parts
-    constexpr bool kHalves = MT == 1 && W::kSuper && !W::kUnits;
+    // sums over a superblock: Q5_K the high and the low halves' apart, Q4_K one
+    constexpr uint32_t kSums = MT == 1 && W::kSuper && !W::kUnits ? (T == T_Q5_K ? 2u : 1u) : 0u;
+    f32x16 acc[MT][2], sum[2][2];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = f32x16{};
     float dcur[2] = {1.0f, 1.0f};
@@ -627,25 +630,27 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
                         acc[m][0] = mfma(hi, b[0][h], acc[m][0]);
                         acc[m][1] = mfma(hi, b[1][h], acc[m][1]);
                     }
-            } else if constexpr (kHalves) {
-                // low and high of one fragment, then of the other; in the superblock's last step
-                // both low ones first, whose sums go into the accumulator while the high ones end
+            } else if constexpr (kSums) {
+                // low and high of one fragment, then of the other; with two sums, in the
+                // superblock's last step both low ones first, so that their sums go into the
+                // accumulator while the high products end
 #pragma unroll
                 for (uint32_t k = 0; k < 4; ++k) {
-                    const uint32_t h = j == 7u ? k & 1u : k / 2u, p = j == 7u ? k < 2u : !(k & 1u);
+                    const bool lows = kSums == 2u && j == 7u;
+                    const uint32_t h = lows ? k & 1u : k / 2u, p = lows ? k < 2u : !(k & 1u), q = p & (kSums - 1u);
                     const f16x8 f = afrag(buf, 0u, p, h);
 #pragma unroll
                     for (uint32_t i = 0; i < 2; ++i)
-                        half[i][p] = mfma(f, b[i][h], j == 0u && h == 0u ? f32x16{} : half[i][p]);
+                        sum[i][q] = mfma(f, b[i][h], j == 0u && k < kSums ? f32x16{} : sum[i][q]);
                 }
                 if (j == 7u) {
 #pragma unroll
-                    for (uint32_t q = 0; q < 2; ++q)
+                    for (uint32_t q = 0; q < kSums; ++q)
 #pragma unroll
                         for (uint32_t i = 0; i < 2; ++i)
 #pragma unroll
                             for (uint32_t r = 0; r < 16; ++r)
-                                acc[0][i][r] = __builtin_fmaf(hd[i].d, half[i][1u - q][r], acc[0][i][r]);
+                                acc[0][i][r] = __builtin_fmaf(hd[i].d, sum[i][kSums - 1u - q][r], acc[0][i][r]);
                 }
             } else {
 #pragma unroll
@@ -690,9 +695,9 @@ __device__ __forceinline__ void gemm_tile(const MoePrefillArgs& a, const TileRef
             load_act((j + 1u) % NS, s + 1u + NS);
             if (j == 4u) store_sums(sbuf ^ 1u);
             __syncthreads();
-            // Q4_K: keeps the next step's decoding behind this one's products (without it 6
-            // registers spill; Q5_K has none to spare either way and is 4% slower with it)
-            if constexpr (kHalves && T == T_Q4_K) __builtin_amdgcn_sched_barrier(0);
+            // Q4_K: keeps the next step's decoding behind this one's products (8 registers
+            // spill without; Q5_K does not spill and is 4% slower with it)
+            if constexpr (kSums == 1u) __builtin_amdgcn_sched_barrier(0);
         }
     }
 
