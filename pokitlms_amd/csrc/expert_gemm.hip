@@ -18,7 +18,7 @@
 // as whole lines through LDS, fragments read half a step ahead with a barrier
 // every second step, and both: the same gate/up time, slower down.)  Error against
 // float64 on the same inputs, before and after: Q4_K/Q6_K 3.8e-6 -> 7.8e-7,
-// Q6_K 9.7e-7 -> 3.6e-7, Q5_K 4.4e-7 -> 3.6e-7, Q8_0 4.4e-7 -> 3.0e-7, Q4_0
+// Q6_K 9.7e-7 -> 3.6e-7, Q5_K 4.4e-7 -> 3.7e-7, Q8_0 4.4e-7 -> 3.0e-7, Q4_0
 // 4.4e-7 -> 2.9e-7, Q4_1 4.6e-7 -> 4.0e-7.
 #include <math.h>
 
